@@ -68,3 +68,73 @@ def test_wide_gemv_argmax(ctx, quant, rows, k):
         # the winner's bytes again at the end of the tensor: the first wins
         rb = w.size // rows
         wd[(rows - 1) * rb:] = wd[idx * rb:(idx + 1) * rb].clone()
+
+
+def rows_of(quant, q, d_bits):
+    """Plain block bytes of the integer quants q [rows][k], one fp16 scale."""
+    rows, k = q.shape
+    b = q.reshape(rows, k // 32, 32)
+    if quant == Q4_0:
+        u = (b + 8).astype(np.uint8)
+        body = u[..., :16] | (u[..., 16:] << 4)
+    else:
+        body = b.astype(np.int8).view(np.uint8)
+    w = np.empty((rows, k // 32, 2 + body.shape[-1]), np.uint8)
+    w[..., :2] = np.frombuffer(np.uint16(d_bits).tobytes(), np.uint8)
+    w[..., 2:] = body
+    return w.reshape(-1)
+
+
+def wide(ctx, x, w, rows, k, quant, il):
+    if il == 4:
+        w = synth.interleave_x4(w, rows, k, quant)
+    y = torch.empty(rows, dtype=torch.float32, device="cuda")
+    ctx.linear_dev(torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda(), y, k, rows, quant, il)
+    return y.cpu().numpy()
+
+
+# plain rows, and X4 groups of in_dims that the segment kernel does not take
+FORMS = [(1, 9, 480), (1, 33, 11008), (4, 8, 96), (4, 12, 14400)]
+
+
+@pytest.mark.parametrize("quant", [Q4_0, Q8_0])
+@pytest.mark.parametrize("il,rows,k", FORMS)
+def test_wide_gemv_sums_the_products_alone(ctx, quant, il, rows, k):
+    """Activations with a large common part and quants of +1, -1 in turn:
+    every partial sum of the products x (d q) is an integer below 2^24 and the
+    result exact, while a sum of x with offset quants (8 or 128 times the
+    common part) would round."""
+    rng = np.random.default_rng(k + quant)
+    x = (2.0 ** 20 + rng.integers(0, 64, k)).astype(np.float32)
+    q = np.empty((rows, k), np.int64)
+    q[:, 0::2] = rng.choice([-1, 1], size=(rows, 1))
+    q[:, 1::2] = -q[:, :1]
+    want = (q @ x.astype(np.float64)).astype(np.float32)
+    got = wide(ctx, x, rows_of(quant, q, 0x3C00), rows, k, quant, il)
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("quant", [Q4_0, Q8_0])
+@pytest.mark.parametrize("il,rows,k", FORMS)
+def test_wide_gemv_infinite_and_huge_activations(ctx, quant, il, rows, k):
+    """An infinite activation gives +-Inf by its quant's sign, NaN where the
+    quant is 0; activations of 1e37 stay finite while their products do."""
+    rng = np.random.default_rng(2 * k + quant)
+    top = 7 if quant == Q4_0 else 127
+    q = rng.integers(-top, top + 1, (rows, k))
+    at = k // 2 + 1
+    q[:3, at] = (5, -5, 0)
+    x = synth.activations(rng, k)
+    w = rows_of(quant, q, 0x0C00)  # d = 2^-12
+    xi = x.copy()
+    xi[at] = np.inf
+    got = wide(ctx, xi, w, rows, k, quant, il)
+    s = np.sign(q[:, at])
+    assert np.array_equal(got[s != 0], np.where(s[s != 0] > 0, np.float32(np.inf), np.float32(-np.inf)))
+    assert np.all(np.isnan(got[s == 0]))
+    xh = (np.float32(1e37) * np.sign(x)).astype(np.float32)
+    ref = q @ xh.astype(np.float64) * 2.0 ** -12
+    got = wide(ctx, xh, w, rows, k, quant, il).astype(np.float64)
+    # an fp32 sum of k products: k roundings of at most sum |x d q| * 2^-24
+    bound = k * 2.0 ** -24 * np.sum(np.abs(q * xh.astype(np.float64)), 1) * 2.0 ** -12
+    assert np.all(np.isfinite(got)) and np.all(np.abs(got - ref) <= bound)

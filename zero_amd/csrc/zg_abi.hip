@@ -419,7 +419,8 @@ zg_status zg::run_linear(zg_ctx* ctx, const float* x, const uint8_t* w, float* y
   g.il = (int)il;
   g.epi = epi;
   if (kq_path_ok(qt, il, k, w, xin)) return hip_check(ctx, launch_gemv_kq(g, st), "gemv_kq launch");
-  if (gemv_wide_ok(qt, (int)il, k, w, xin)) return hip_check(ctx, launch_gemv_wide(g, st), "gemv_wide launch");
+  if (gemv_wide_ok(qt, (int)il, k, w, xin))
+    return hip_check(ctx, launch_gemv_wide(g, !pair_path_ok(qt, il, k, n, w, xin), st), "gemv_wide launch");
   return hip_check(ctx, launch_gemv_generic(g, st), "gemv_generic launch");
 }
 

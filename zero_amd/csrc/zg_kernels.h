@@ -120,8 +120,10 @@ size_t gemv_x4_lds_bytes(uint32_t qt, int k);
 hipError_t launch_gemv_generic(const GenericArgs& a, hipStream_t st);
 // Q4_0 / Q8_0 rows or X4 groups of any in_dim and row count
 // (zg_gemv_wide.hip); w 2-byte (plain) or 8-byte (X4) aligned, x 16-byte.
+// direct: an X4 block's terms as x (d q), the generic kernel's, in place of
+// the X4 kernels' d (sum(u x) - offset sum(x)); plain rows are always direct.
 bool gemv_wide_ok(uint32_t qt, int il, size_t k, const void* w, const void* x);
-hipError_t launch_gemv_wide(const GenericArgs& a, hipStream_t st);
+hipError_t launch_gemv_wide(const GenericArgs& a, bool direct, hipStream_t st);
 hipError_t launch_dequant(const DequantArgs& a, bool pair_path, hipStream_t st);
 // Q4_K / Q6_K fast path (row-major superblocks, in_dim a multiple of 256
 // and at most kMaxKqK so that x and its 16-element sums fit 64 KiB of LDS).
