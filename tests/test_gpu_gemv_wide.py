@@ -138,3 +138,24 @@ def test_wide_gemv_infinite_and_huge_activations(ctx, quant, il, rows, k):
     # an fp32 sum of k products: k roundings of at most sum |x d q| * 2^-24
     bound = k * 2.0 ** -24 * np.sum(np.abs(q * xh.astype(np.float64)), 1) * 2.0 ** -12
     assert np.all(np.isfinite(got)) and np.all(np.abs(got - ref) <= bound)
+
+
+# one wide launch of the segments; wide segments around one that the segment
+# kernel takes (more than 4,096 rows, or 2,048 above in_dim 2560); an in_dim
+# that only the wide kernel takes (a launch per segment)
+@pytest.mark.parametrize("quant,k,ns", [(Q4_0, 2176, (8, 4, 2052)), (Q8_0, 5056, (1028, 4, 512)), (Q4_0, 5056, (4, 2048)),
+                                        (Q4_0, 2560, (4, 4096)), (Q4_0, 2176, (4, 4100, 12)), (Q8_0, 2624, (2052, 8)),
+                                        (Q8_0, 96, (8, 12, 4))])
+def test_fused_call_gives_the_bits_of_single_calls(ctx, quant, k, ns):
+    rng = np.random.default_rng(k + quant)
+    x = torch.from_numpy(synth.activations(rng, k)).cuda()
+    ws = [torch.from_numpy(synth.weight(rng, quant, n, k, 4)).cuda() for n in ns]
+    one = [torch.empty(n, dtype=torch.float32, device="cuda") for n in ns]
+    for w, y, n in zip(ws, one, ns):
+        ctx.linear_dev(x, w, y, k, n, quant, 4)
+    y = torch.full((sum(ns) + 4,), -7.0, dtype=torch.float32, device="cuda")
+    parts = list(torch.split(y[:-4], ns))
+    ctx.linear_fused_dev(x, [(w, p, n, quant, 4) for w, p, n in zip(ws, parts, ns)], k)
+    got = y.cpu().numpy()
+    assert np.array_equal(got[:-4].view(np.uint32), torch.cat(one).cpu().numpy().view(np.uint32))
+    assert np.all(got[-4:] == -7.0)

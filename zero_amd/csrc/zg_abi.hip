@@ -303,20 +303,27 @@ zg_status zg::check_shape(zg_ctx* ctx, uint32_t qt, uint32_t il, size_t k, size_
   return ZG_OK;
 }
 
+// X4 groups without a prologue whose in_dim is outside the strip kernel's
+// range take the wide kernel up to 2,048 rows (4,096 for in_dims up to 2560),
+// else the segment-streaming kernel.  Q4_0X4, wide / segment, us: 2048x2880
+// 3.5 / 5.1, 2048x9728 5.9 / 9.1, 4096x2176 3.8 / 5.6, 4096x5056 6.1 / 6.9,
+// 8192x5056 9.9 / 9.3, 16384x5056 17.7 / 13.7; Q8_0X4 2048x5056 5.4 / 7.9,
+// 16384x2880 15.6 / 13.1: taller tensors hide the segment kernel's start, and
+// the wide kernel's partial last round of chunks then costs more.  The rule
+// takes the whole tensor's rows, and a fused call asks it for each of its
+// segments, so that row ranges and fused calls give the bits of the full
+// call; the line lies where three tensors in one launch still win (Q4_0X4,
+// k = 5056: 3 x 2048 rows 7.9 / 8.4, 3 x 4096 rows 14.3 / 11.3).
+static bool wide_x4_ok(uint32_t qt, uint32_t il, size_t k, size_t n, const void* w, const void* x) {
+  return il == 4 && n <= (k <= 2560 ? 4096u : 2048u) && !strip_path_ok((int)k) && gemv_wide_ok(qt, 4, k, w, x);
+}
+
 // One GEMV (optionally a row range, residual or argmax epilogue).
 zg_status zg::run_linear(zg_ctx* ctx, const float* x, const uint8_t* w, float* y, size_t k, size_t n, uint32_t qt,
                          uint32_t il, size_t start, size_t end, int epi, const float* resid, uint64_t* best,
                          int pro, const float* norm_w, float eps, hipStream_t st, uint32_t gemv_flags) {
   if (start >= end) return ZG_OK;
-  // X4 groups without a prologue whose in_dim is outside the strip kernel's
-  // range take the wide kernel up to 48 MB of weights: 4096x9728 Q4_0X4 8.3
-  // against 9.6 us on the segment-streaming kernel, 4096x2176 3.8 against
-  // 5.6 us, 32768x2176 16.0 against 16.8 us; larger tensors stream better in
-  // segments (16384x8704 23.6 against 25.3 us, Q8_0X4 32768x2176 20.2 against
-  // 21.3 us).  The rule takes the whole tensor's rows, so that a row range
-  // runs the kernel of the full call.
-  const bool wide_x4 = il == 4 && pro == PRO_PLAIN && !(gemv_flags & kGemvStream) && !strip_path_ok((int)k) &&
-                       tensor_bytes(qt, n, k) <= ((size_t)48 << 20) && gemv_wide_ok(qt, 4, k, w, x);
+  const bool wide_x4 = pro == PRO_PLAIN && !(gemv_flags & kGemvStream) && wide_x4_ok(qt, il, k, n, w, x);
   if (!wide_x4 && pair_path_ok(qt, il, k, n, w, x)) {
     const size_t gbytes = (k / 32) * (qt == ZG_Q4_0 ? 72 : 136);
     const size_t g0 = start / 4, g1 = (end + 3) / 4;
@@ -546,6 +553,35 @@ zg_status zg::run_fused(zg_ctx* ctx, const float* x, const FusedDev* segs, size_
   const bool plain = !pair && fused_plain_ok(x, segs, nseg, k, pro);
   if (epi == EPI_SWIGLU && !((pair || plain) && nseg == 2 && segs[0].n == segs[1].n))
     return set_error(ctx, ZG_ERR_INVALID_ARG, "swiglu fusion needs two equal Q4_0/Q8_0 segments on a one-launch path");
+  if (pair && pro == PRO_PLAIN && epi == EPI_STORE) {
+    // the segments that a call of their own would give to the wide kernel in
+    // one launch of it, the others in one of the segment kernel
+    FusedDev rest[3];
+    size_t nrest = 0, nwide = 0;
+    GenericArgs g{};
+    for (size_t i = 0; i < nseg; i++) {
+      if (!wide_x4_ok(segs[i].qt, segs[i].il, k, segs[i].n, segs[i].w, x)) {
+        rest[nrest++] = segs[i];
+        continue;
+      }
+      g.seg_w[nwide] = segs[i].w;
+      g.seg_y[nwide] = segs[i].y;
+      g.row_hi += segs[i].n;
+      g.seg_end[nwide++] = (uint32_t)g.row_hi;
+    }
+    if (nwide) {
+      for (size_t i = nwide; i < 3; i++) g.seg_end[i] = (uint32_t)g.row_hi;
+      g.x = x;
+      g.k = k;
+      g.qt = segs[0].qt;
+      g.il = 4;
+      g.epi = EPI_STORE;
+      g.nseg = (int)nwide;
+      zg_status s = hip_check(ctx, launch_gemv_wide_segs(g, st), "fused gemv_wide launch");
+      if (s || !nrest) return s;
+      return run_fused(ctx, x, rest, nrest, k, pro, norm_w, eps, epi, st);
+    }
+  }
   if (pair || plain) {
     GemvArgs a{};
     a.nseg = (int)nseg;

@@ -80,7 +80,8 @@ struct GenericArgs {
   const float* norm_w;
   float eps;
   const uint8_t* w_up;
-  // Q4_K strip kernel, EPI_STORE: nseg > 1 concatenates up to 3 projections
+  // Q4_K strip kernel and the wide kernel's segmented launch, EPI_STORE:
+  // nseg > 1 concatenates up to 3 projections
   // of the same x (rows [seg_end[i-1], seg_end[i]) are segment i's rows 0..,
   // weights seg_w[i], outputs seg_y[i]); w / y / row range are then unused
   int nseg;
@@ -124,6 +125,9 @@ hipError_t launch_gemv_generic(const GenericArgs& a, hipStream_t st);
 // the X4 kernels' d (sum(u x) - offset sum(x)); plain rows are always direct.
 bool gemv_wide_ok(uint32_t qt, int il, size_t k, const void* w, const void* x);
 hipError_t launch_gemv_wide(const GenericArgs& a, bool direct, hipStream_t st);
+// whole X4 tensors of one x in one launch (GenericArgs' segments, rows 0 to
+// their total; EPI_STORE, the X4 kernels' form of the terms)
+hipError_t launch_gemv_wide_segs(const GenericArgs& a, hipStream_t st);
 hipError_t launch_dequant(const DequantArgs& a, bool pair_path, hipStream_t st);
 // Q4_K / Q6_K fast path (row-major superblocks, in_dim a multiple of 256
 // and at most kMaxKqK so that x and its 16-element sums fit 64 KiB of LDS).
