@@ -327,6 +327,12 @@ size_t zg_model_first_nonfinite(const zg_model *m, char *buf, size_t cap);
  * Every kernel still runs to its end.  layer < 0 restores the stores (the
  * default).  Affects only layers decoded by the fused launch. */
 zg_status zg_model_test_drop_qkv_stores(zg_model *m, int32_t layer);
+/* The fused Q|K|V + attention launches of the step at position pos: how many
+ * workgroups of one launch wait for its GEMV (0: no layer has such a launch),
+ * and how many workgroups of the launch the device holds at once (the fewest
+ * over the layers).  No counterpart in the reference; the waits end while the
+ * waiting workgroups of all launches in flight are fewer than the slots. */
+zg_status zg_model_step_waiters(const zg_model *m, uint32_t pos, uint32_t *waiters, uint32_t *slots);
 
 /* Batched prefill.  No counterpart in the reference, which runs the prompt
  * token by token through forward_single_token_avx512

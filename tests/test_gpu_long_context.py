@@ -2,6 +2,8 @@
 attention splits and, in the fused Q|K|V + attention launch, longer rounds):
 greedy tokens and hidden states against the oracle across it, and the same
 bits from single steps and from the device loop."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -35,4 +37,25 @@ def test_decode_across_the_long_context_switch(ctx, zo, hidden, lin, n_q, n_kv, 
     finally:
         gm.close()
         om.close()
+        ctx.clear()
+
+
+# (query heads, KV heads, head dim): splits of the steps past the switch
+@pytest.mark.parametrize("n_q,n_kv,hd,splits", [(16, 8, 128, 8), (22, 11, 128, 8), (24, 8, 128, 6), (32, 8, 128, 6),
+                                                (31, 31, 64, 8), (32, 8, 64, 6)])
+def test_waiting_workgroups_leave_slots_for_the_gemv(ctx, n_q, n_kv, hd, splits):
+    """The attention workgroups of the fused launch wait for its GEMV: those of
+    four such launches at once (four contexts) have to be fewer than the
+    device holds, or the launch keeps the base form's six splits."""
+    cfg = synth.ModelConfig(n_layers=1, hidden=2048, ffn=512, n_q_heads=n_q, n_kv_heads=n_kv, head_dim=hd, vocab_padded=512,
+                            vocab_real=500, max_ctx=720)
+    gm = GpuModel(ctx, synth.random_model(cfg, seed=n_q))
+    try:
+        for pos in (0, 639, 640, 719):
+            w, slots = C.c_uint32(), C.c_uint32()
+            ctx.check(ctx.lib.zg_model_step_waiters(gm.h, pos, C.byref(w), C.byref(slots)))
+            assert w.value == n_q * (splits if pos >= 640 else 6)
+            assert 4 * w.value < slots.value, pos
+    finally:
+        gm.close()
         ctx.clear()

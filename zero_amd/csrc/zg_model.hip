@@ -173,12 +173,14 @@ constexpr int kAttnDecodeSplits = ZG_ATTN_SPLITS;
 static_assert(kAttnDecodeSplits >= 1 && kAttnDecodeSplits <= kAttnSplits, "decode splits within the merge's capacity");
 // Steps at positions from kLongPos on take the long-context launches: as many
 // splits as the merge holds and, in the fused launch, rounds of 128 rows
-// instead of 64 (fewer dependent memory round trips per split, at 172 VGPRs,
+// instead of 64 (fewer dependent memory round trips per split, at 166 VGPRs,
 // which fewer workgroups share a CU with).  Qwen3-1.7B shape, Q4_0X4, us per
-// step: at 1,500 888 -> 800, at 2,000 964 -> 859, at 768 737 -> 712; at 512 694
+// step: at 1,500 887 -> 817, at 2,000 961 -> 884, at 768 740 -> 714; at 512 694
 // against 700 and at 64 636 against 680, so shorter contexts keep six splits
-// and 64-row rounds.  (Eight splits with 64-row rounds: 841 at 1,500; six with
-// 128-row ones: 842; with 192-row ones: 890.)
+// and 64-row rounds.  (At 172 VGPRs, two workgroups per CU, whose slots four
+// launches' waiting workgroups could fill: 800 at 1,500; then eight splits
+// with 64-row rounds 841, six with 128-row ones 842, with 192-row ones 890.)  A model
+// whose waiting workgroups would not fit (step_waiters_fit) keeps the base form.
 constexpr uint32_t kLongPos = 640;
 
 // Decode attention, flash-decoding over splits: grid (query heads, splits),
@@ -265,8 +267,8 @@ __device__ __forceinline__ void attn_split_body(AttnArgs a, int qh, int sp, int 
 #pragma unroll
     for (int p = 0; p < NP; p++) {
       if (rb + p * PASS < n_t) {
-        const int tk = min(rb + p * PASS + wave * RPW + r, n_t - 1);
-        const size_t ko = (size_t)(c0 + tk) * rowf4 + kvh * F4;
+        const int t0 = rb + p * PASS + wave * RPW;
+        const size_t ko = (size_t)(c0 + t0 + min(r, n_t - 1 - t0)) * rowf4 + kvh * F4;
 #pragma unroll
         for (int i = 0; i < CPL; i++) kr[p][i] = K4[ko + sl + LPR * i];
 #pragma unroll
@@ -379,11 +381,10 @@ __device__ __forceinline__ void attn_split_body(AttnArgs a, int qh, int sp, int 
     for (int p = 0; p < NP; p++) {
       sc[p] = -INFINITY;
       if (rb + p * PASS < n_t) {
-        const int t = rb + p * PASS + wave * RPW + r;
-        float4 kk[CPL];
-#pragma unroll
-        for (int i = 0; i < CPL; i++) kk[i] = kr[p][i];
-        if (c0 + t == pos) {
+        // (this wave's first row in scalar registers, the lane's row r past it)
+        const int t0 = rb + p * PASS + wave * RPW;
+        float4(&kk)[CPL] = kr[p];
+        if (r == pos - c0 - t0) {
 #pragma unroll
           for (int i = 0; i < CPL; i++) kk[i] = reinterpret_cast<const float4*>(krow)[sl + LPR * i];
         }
@@ -398,7 +399,7 @@ __device__ __forceinline__ void attn_split_body(AttnArgs a, int qh, int sp, int 
         d += dpp_f32<0xB1>(d);   // quad_perm [1,0,3,2]
         d += dpp_f32<0x4E>(d);   // quad_perm [2,3,0,1]
         d += dpp_f32<0x141>(d);  // row_half_mirror: the 8 lanes of the row
-        sc[p] = t < n_t ? d * a.scale : -INFINITY;
+        sc[p] = r < n_t - t0 ? d * a.scale : -INFINITY;
         nan_score = nan_score || __builtin_isnan(sc[p]);
         cmax = fmaxf(cmax, sc[p]);
       }
@@ -468,7 +469,10 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_split_kernel(AttnArgs a)
 // groups per batch).  The attention workgroups come first, so they are
 // dispatched first: they issue their K/V cache loads while the GEMV runs,
 // then poll the GEMV's rows, each stored once with this step and layer's
-// tag (the GEMV never waits, so every poll ends; it is also bounded).
+// tag.  The GEMV never waits, so every poll ends once the GEMV's workgroups
+// find slots: the waiting workgroups, of every launch that can be in flight
+// with this one, have to be fewer than the chip holds (step_waiters_fit; the
+// polls are also bounded, and then fail the step).
 // One launch instead of two, and the attention's cache reads overlap the
 // GEMV.  A counter that every batch incremented serialised the 512 atomics
 // of a step on one line (19 vs 8.8 us for the two kernels).
@@ -478,8 +482,12 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_split_kernel(AttnArgs a)
 constexpr int kFusedAttnPasses = ZG_FUSED_ATTN_PASSES;
 constexpr int kFusedAttnPassesLong = 4;
 
+// The long form is held to three workgroups per CU at head_dim 128 (166
+// VGPRs; 172 with a lane's row numbers and copies of the K row in vector
+// registers, two per CU), so that its waiting workgroups share 768 slots; at
+// head_dim 64, and in the base forms, four and more fit by themselves.
 template <uint32_t QT, int IL, int HD, int NP>
-__global__ __launch_bounds__(256) void qkv_attn_kernel(GemvArgs ga, AttnArgs aa, int n_attn) {
+__global__ __launch_bounds__(256, NP == kFusedAttnPassesLong && HD == 128 ? 3 : 1) void qkv_attn_kernel(GemvArgs ga, AttnArgs aa, int n_attn) {
   const int b = blockIdx.x;
   if (b < n_attn) {
     const int nq = n_attn / aa.nsplit;
@@ -1166,6 +1174,49 @@ static zg_status head_argmax(zg_model* m, const float* x, hipStream_t st) {
                     d.rms_eps, st, kGemvStream);
 }
 
+// The qkv_attn_kernel of Q4_K rows, or X4 / split-scale X4 Q4_0 / Q8_0
+// (plain-row Q4_0 / Q8_0 projections are interleaved at model creation).
+typedef void (*QkvAttnFn)(GemvArgs, AttnArgs, int);
+constexpr size_t kQkvAttnShm = 2 * 4 * 2 * 16 * sizeof(float);  // the strip body's [2][4 waves][2 groups][16] partials
+template <int HD, int NP>
+static QkvAttnFn qkv_attn_fn_hd(uint32_t qt, uint32_t il) {
+  if (qt == ZG_Q4K) return qkv_attn_kernel<Q4K, 1, HD, NP>;
+  if (qt == ZG_Q4_0 && il == 5) return qkv_attn_kernel<Q4_0, 5, HD, NP>;
+  if (qt == ZG_Q4_0 && il == 4) return qkv_attn_kernel<Q4_0, 4, HD, NP>;
+  if (qt == ZG_Q8_0 && il == 5) return qkv_attn_kernel<Q8_0, 5, HD, NP>;
+  if (qt == ZG_Q8_0 && il == 4) return qkv_attn_kernel<Q8_0, 4, HD, NP>;
+  return nullptr;
+}
+static QkvAttnFn qkv_attn_fn(uint32_t qt, uint32_t il, int hd, bool lng) {
+  if (hd == 128)
+    return lng ? qkv_attn_fn_hd<128, kFusedAttnPassesLong>(qt, il) : qkv_attn_fn_hd<128, kFusedAttnPasses>(qt, il);
+  return lng ? qkv_attn_fn_hd<64, kFusedAttnPassesLong>(qt, il) : qkv_attn_fn_hd<64, kFusedAttnPasses>(qt, il);
+}
+
+// Workgroups of layer L's fused launch that the device holds at once; 0 when
+// that cannot be told.
+static size_t qkv_attn_slots(const zg_model* m, const ZLayer& L, bool lng) {
+  const auto fn = qkv_attn_fn(L.qt[ZG_PROJ_Q], L.il[ZG_PROJ_Q], (int)m->d.head_dim, lng);
+  int n = 0;
+  if (!fn || hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void*>(fn), 256, kQkvAttnShm) !=
+                 hipSuccess || n <= 0) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return (size_t)n * (size_t)m->cus;
+}
+
+// Whether the waiting workgroups of the long form leave slots for the GEMVs
+// when kStepsInFlight contexts run such a launch at once (one per hardware
+// queue of a process).  Workgroups go to the XCDs in turn and both counts are
+// multiples of the eight XCDs, so fewer in all is fewer on each.  16 query
+// heads of 128: 4 x 128 of 768 slots; 24 and more heads keep the base form,
+// whose six splits have 1,024 slots.
+constexpr size_t kStepsInFlight = 4;
+static bool step_waiters_fit(const zg_model* m, const ZLayer& L) {
+  return kStepsInFlight * m->d.n_q_heads * kAttnSplits < qkv_attn_slots(m, L, true);
+}
+
 // Layer l's Q|K|V GEMV (rmsnorm prologue) and decode attention as one
 // qkv_attn_kernel launch; aa holds the attention arguments.
 static zg_status run_qkv_attn(zg_model* m, uint32_t l, const ZLayer& L, AttnArgs aa, bool lng, hipStream_t st) {
@@ -1207,34 +1258,10 @@ static zg_status run_qkv_attn(zg_model* m, uint32_t l, const ZLayer& L, AttnArgs
   aa.tag_add = l;
   const int n_attn = (int)d.n_q_heads * aa.nsplit;
   const dim3 grid((unsigned)(n_attn + gb / 2)), block(256);
-  const size_t shm = 2 * 4 * 2 * 16 * sizeof(float);  // the strip body's [2][4 waves][2 groups][16] partials
   const uint32_t qt = L.qt[ZG_PROJ_Q], il = L.il[ZG_PROJ_Q];
-#define ZG_QKV_ATTN_NP(QT, IL, HDV, NP) \
-  hipLaunchKernelGGL((qkv_attn_kernel<QT, IL, HDV, NP>), grid, block, shm, st, ga, aa, n_attn)
-#define ZG_QKV_ATTN(QT, IL, HDV)                               \
-  do {                                                         \
-    if (lng) ZG_QKV_ATTN_NP(QT, IL, HDV, kFusedAttnPassesLong); \
-    else ZG_QKV_ATTN_NP(QT, IL, HDV, kFusedAttnPasses);         \
-  } while (0)
-  // Q4_K rows, or X4 / split-scale X4 Q4_0 / Q8_0 (plain-row Q4_0 / Q8_0
-  // projections are interleaved at model creation)
-  if (qt != ZG_Q4K && il != 4 && il != 5)
-    return set_error(m->ctx, ZG_ERR_UNSUPPORTED_QUANT, "qkv+attention: plain-row Q4_0/Q8_0");
-  if (HD == 128) {
-    if (qt == ZG_Q4K) ZG_QKV_ATTN(Q4K, 1, 128);
-    else if (qt == ZG_Q4_0 && il == 5) ZG_QKV_ATTN(Q4_0, 5, 128);
-    else if (qt == ZG_Q4_0) ZG_QKV_ATTN(Q4_0, 4, 128);
-    else if (il == 5) ZG_QKV_ATTN(Q8_0, 5, 128);
-    else ZG_QKV_ATTN(Q8_0, 4, 128);
-  } else {
-    if (qt == ZG_Q4K) ZG_QKV_ATTN(Q4K, 1, 64);
-    else if (qt == ZG_Q4_0 && il == 5) ZG_QKV_ATTN(Q4_0, 5, 64);
-    else if (qt == ZG_Q4_0) ZG_QKV_ATTN(Q4_0, 4, 64);
-    else if (il == 5) ZG_QKV_ATTN(Q8_0, 5, 64);
-    else ZG_QKV_ATTN(Q8_0, 4, 64);
-  }
-#undef ZG_QKV_ATTN
-#undef ZG_QKV_ATTN_NP
+  const auto fn = qkv_attn_fn(qt, il, HD, lng);
+  if (!fn) return set_error(m->ctx, ZG_ERR_UNSUPPORTED_QUANT, "qkv+attention: plain-row Q4_0/Q8_0");
+  hipLaunchKernelGGL(fn, grid, block, kQkvAttnShm, st, ga, aa, n_attn);
   return hip_check(m->ctx, hipGetLastError(), "qkv+attention launch");
 }
 
@@ -1799,6 +1826,9 @@ extern "C" zg_status zg_model_create(zg_ctx* ctx, const zg_model_desc* desc, zg_
                    il[ZG_PROJ_Q] == il[ZG_PROJ_V] && H == 2048 && (d.head_dim == 128 || d.head_dim == 64) &&
                    groups / 2 <= (size_t)m->cus * 4;
     }
+    // no long form unless its waiting workgroups fit in every layer
+    for (const ZLayer& L : m->layers)
+      if (m->nsplit_long && L.qkv_attn && !step_waiters_fit(m, L)) m->nsplit_long = 0;
     m->head_norm =
         rmsnorm_fused_ok(d.head_type, m->d.head_interleave, H, d.vocab_padded, m->head, m->hidden, EPI_ARGMAX);
   }
@@ -1950,6 +1980,20 @@ extern "C" zg_status zg_model_test_drop_qkv_stores(zg_model* m, int32_t layer) {
                           "drop hook upload");
   if (!s) s = hip_check(m->ctx, hipStreamSynchronize(m->ctx->stream), "drop hook upload");
   return s;
+}
+
+extern "C" zg_status zg_model_step_waiters(const zg_model* m, uint32_t pos, uint32_t* waiters, uint32_t* slots) {
+  if (!m || !waiters || !slots || pos >= m->d.max_ctx) return ZG_ERR_INVALID_ARG;
+  hipSetDevice(m->ctx->device);
+  const bool lng = is_long(m, pos);
+  *waiters = *slots = 0;
+  for (const ZLayer& L : m->layers) {
+    if (!L.qkv_attn) continue;
+    const uint32_t n = (uint32_t)qkv_attn_slots(m, L, lng);
+    *slots = *waiters && *slots < n ? *slots : n;
+    *waiters = m->d.n_q_heads * (uint32_t)(lng ? m->nsplit_long : m->nsplit);
+  }
+  return ZG_OK;
 }
 
 extern "C" size_t zg_model_first_nonfinite(const zg_model* m, char* buf, size_t cap) {
