@@ -334,6 +334,15 @@ zg_status zg_model_test_drop_qkv_stores(zg_model *m, int32_t layer);
  * waiting workgroups of all launches in flight are fewer than the slots. */
 zg_status zg_model_step_waiters(const zg_model *m, uint32_t pos, uint32_t *waiters, uint32_t *slots);
 
+/* Rows that the batched prefill's buffers hold now (0 before its first call):
+ * the longest prompt so far in steps of 512, at most 2048 and max_ctx; fewer
+ * where that did not fit in device memory, down to 512.  Longer prompts run
+ * in chunks of so many rows. */
+size_t zg_model_prefill_rows(const zg_model *m);
+/* Failure-path test hook: row buffers of more than `rows` rows are treated as
+ * not fitting in device memory (0, the default: none are). */
+zg_status zg_model_test_prefill_fit(zg_model *m, size_t rows);
+
 /* Batched prefill.  No counterpart in the reference, which runs the prompt
  * token by token through forward_single_token_avx512
  * (kernel/src/inference.rs:1188-1330); this is the M >= 64 prefill of the

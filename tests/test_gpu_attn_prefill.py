@@ -99,3 +99,36 @@ def test_prefill_across_a_chunk_boundary(ctx):
     finally:
         gm.close()
         ctx.clear()
+
+
+def test_prefill_row_buffers_follow_the_prompt_and_the_memory(ctx):
+    """The row buffers hold the longest prompt so far in steps of 512 rows;
+    where they do not fit, fewer rows run the prompt in more chunks with the
+    same bits, down to 512, below which the call fails and a later one runs."""
+    cfg = synth.ModelConfig(n_layers=2, hidden=256, ffn=256, n_q_heads=4, n_kv_heads=2, head_dim=64, vocab_padded=512,
+                            vocab_real=500, max_ctx=2100)
+    gm = GpuModel(ctx, synth.random_model(cfg, seed=9))
+    rows, fit = ctx.lib.zg_model_prefill_rows, ctx.lib.zg_model_test_prefill_fit
+    try:
+        prompt = synth.prompt(6, 2081, cfg.vocab_real)
+        assert fit(gm.h, 100) == _lib.ZG_OK and rows(gm.h) == 0
+        with pytest.raises(ZgError) as ei:
+            gm.prefill(prompt[:10])
+        assert ei.value.code == _lib.ZG_ERR_OUT_OF_MEMORY and rows(gm.h) == 0
+        assert fit(gm.h, 0) == _lib.ZG_OK
+        seen = []
+        for n in (10, 512, 513, 10, 1500, 2081):
+            gm.reset()
+            want = gm.prefill(prompt[:n], want_hidden=True)
+            seen.append(rows(gm.h))
+        assert seen == [512, 512, 1024, 1024, 1536, 2048]
+        gm.close()
+        ctx.clear()
+        gm = GpuModel(ctx, synth.random_model(cfg, seed=9))
+        assert fit(gm.h, 1000) == _lib.ZG_OK
+        got = gm.prefill(prompt, want_hidden=True)
+        assert rows(gm.h) == 512
+        assert got[0] == want[0] and got[1] == want[1] and np.array_equal(got[2], want[2])
+    finally:
+        gm.close()
+        ctx.clear()

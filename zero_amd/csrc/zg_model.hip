@@ -1020,9 +1020,11 @@ struct zg_model {
   // which returns the step's final hidden state)
   // ([1]: the long-context forms, positions from kLongPos on)
   hipGraphExec_t g_prefill[2] = {}, g_step[2] = {}, g_step_host[2] = {};
-  // batched prefill: row buffers for chunks of up to pf_cap tokens,
-  // allocated on first use
+  // batched prefill: row buffers for chunks of up to pf_cap tokens (pf_mem
+  // holds them all), allocated by the first call and grown by longer prompts
   size_t pf_cap = 0;
+  void* pf_mem = nullptr;
+  size_t pf_fit = 0;  // test hook: buffers of more rows do not fit (0: none)
   float *pf_x = nullptr, *pf_q = nullptr, *pf_k = nullptr, *pf_v = nullptr;
   float *pf_g = nullptr, *pf_u = nullptr;
   int8_t* pf_qs = nullptr;
@@ -1053,9 +1055,11 @@ enum RowKind : uint8_t { kRowUnknown = 0, kRowDecode = 1, kRowBatched = 2 };
 // prompt of any usual length in one chunk: its GEMMs get more tiles per
 // launch and its attention fewer half-empty last rounds (1,800 tokens of the
 // Qwen3-1.7B shape, Q4_0X4 / Q4_K_M: 17.3 / 21.3 ms, against 22.2 / 29.3 ms
-// in chunks of 512 and 18.8 / 23.3 ms of 1,024); the row buffers take 170 MB
-// at that shape.
+// in chunks of 512 and 18.8 / 23.3 ms of 1,024); the row buffers take 83 KB a
+// row at that shape, in steps of kPrefillStep rows by the longest prompt (42
+// MB up to 512 rows, 170 MB from 1,537 on).
 constexpr size_t kPrefillChunk = 2048;
+constexpr size_t kPrefillStep = 512;
 
 static zg_status model_alloc(zg_model* m, void** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
@@ -1451,32 +1455,62 @@ static zg_status capture(zg_model* m, zg_status (*rec)(zg_model*, hipStream_t, b
   return hip_check(ctx, e, "graph instantiate");
 }
 
-static zg_status prefill_alloc(zg_model* m) {
-  if (m->pf_cap) return ZG_OK;
+// Row buffers for chunks of C rows in one allocation, laid out in turn
+// (sizes only when base is null).  Returns the bytes.
+static size_t prefill_layout(zg_model* m, size_t C, uint8_t* base) {
   const zg_model_desc& d = m->d;
-  const size_t C = d.max_ctx < kPrefillChunk ? d.max_ctx : kPrefillChunk;
   const size_t H = d.hidden, F = d.ffn, qd = (size_t)d.n_q_heads * d.head_dim, kvd = (size_t)d.n_kv_heads * d.head_dim;
   const size_t kmax = std::max(H, std::max(qd, F));
-  zg_status s = ZG_OK;
-  auto al = [&](auto** p, size_t bytes) {
-    if (!s) s = model_alloc(m, reinterpret_cast<void**>(p), bytes);
+  size_t off = 0;
+  auto part = [&](auto** p, size_t bytes) {
+    if (base) *p = reinterpret_cast<std::remove_reference_t<decltype(*p)>>(base + off);
+    off += (bytes + 255) / 256 * 256;
   };
-  al(&m->pf_x, C * H * 4);
-  al(&m->pf_q, C * qd * 4);
-  al(&m->pf_k, C * kvd * 4);
-  al(&m->pf_v, C * kvd * 4);
-  al(&m->pf_g, C * F * 4);
-  al(&m->pf_u, C * F * 4);
-  al(&m->pf_qs, C * kmax);
-  al(&m->pf_qd, C * (kmax / 32) * 2);
+  part(&m->pf_x, C * H * 4);
+  part(&m->pf_q, C * qd * 4);
+  part(&m->pf_k, C * kvd * 4);
+  part(&m->pf_v, C * kvd * 4);
+  part(&m->pf_g, C * F * 4);
+  part(&m->pf_u, C * F * 4);
+  part(&m->pf_qs, C * kmax);
+  part(&m->pf_qd, C * (kmax / 32) * 2);
   if (m->pf_kq) {
-    al(&m->pf_ks, C * kmax);
-    al(&m->pf_k8, C * (kmax / 256) * 4);
-    al(&m->pf_kb, C * (kmax / 32) * 2);
-    al(&m->pf_a, C * qd * 4);
+    part(&m->pf_ks, C * kmax);
+    part(&m->pf_k8, C * (kmax / 256) * 4);
+    part(&m->pf_kb, C * (kmax / 32) * 2);
+    part(&m->pf_a, C * qd * 4);
   }
-  if (!s) m->pf_cap = C;
-  return s;
+  return off;
+}
+
+// Row buffers for a prompt of n rows: the prompt's rows in steps of
+// kPrefillStep, up to a chunk, kept and grown when a longer prompt comes.
+// Where that does not fit, half as many rows and so on down to one step
+// (the prompt then runs in more chunks, with the same bits).
+static zg_status prefill_alloc(zg_model* m, size_t n) {
+  const size_t top = std::min<size_t>(m->d.max_ctx, kPrefillChunk), low = std::min(top, kPrefillStep);
+  size_t C = std::min(top, (n + kPrefillStep - 1) / kPrefillStep * kPrefillStep);
+  if (m->pf_cap >= C) return ZG_OK;
+  if (m->pf_cap) {
+    zg_status s = hip_check(m->ctx, hipStreamSynchronize(m->ctx->stream), "prefill rows sync");
+    if (s) return s;
+    hipFree(m->pf_mem);
+    m->pf_mem = nullptr;
+    m->pf_cap = 0;
+  }
+  for (;; C = std::max(C / 2, low)) {
+    void* p = nullptr;
+    const size_t bytes = prefill_layout(m, C, nullptr);
+    const hipError_t e = m->pf_fit && C > m->pf_fit ? hipErrorOutOfMemory : hipMalloc(&p, bytes);
+    if (e == hipSuccess) {
+      m->pf_mem = p;
+      m->pf_cap = C;
+      prefill_layout(m, C, static_cast<uint8_t*>(p));
+      return hip_check(m->ctx, hipMemsetAsync(p, 0, bytes, m->ctx->stream), "prefill rows clear");
+    }
+    if (C == low) return alloc_failed(m->ctx, e, "prefill rows", bytes);
+    (void)hipGetLastError();
+  }
 }
 
 static bool kq_type(uint32_t t) { return t == ZG_Q4K || t == ZG_Q6K; }
@@ -1578,7 +1612,7 @@ static zg_status prefill_chunk(zg_model* m, const uint32_t* d_tokens, size_t n, 
 static zg_status prefill_run(zg_model* m, size_t off, size_t n, uint32_t pos0, size_t* last_rows) {
   const zg_model_desc& d = m->d;
   hipStream_t st = m->ctx->stream;
-  zg_status s = prefill_alloc(m);
+  zg_status s = prefill_alloc(m, n);
   size_t rows = 0;
   for (size_t c = 0; c < n && !s; c += rows) {
     rows = std::min(m->pf_cap, n - c);
@@ -1853,6 +1887,7 @@ extern "C" void zg_model_destroy(zg_model* m) {
   for (int i = 0; i < 2; i++)
     for (hipGraphExec_t g : {m->g_prefill[i], m->g_step[i], m->g_step_host[i]})
       if (g) hipGraphExecDestroy(g);
+  if (m->pf_mem) hipFree(m->pf_mem);
   for (void* p : m->owned) hipFree(p);
   delete m;  // drops the weight references: copies cleared from the registry are freed here
   if (--ctx->live_models == 0 && ctx->destroy_pending) destroy_context(ctx);
@@ -1982,6 +2017,14 @@ extern "C" zg_status zg_model_test_drop_qkv_stores(zg_model* m, int32_t layer) {
   return s;
 }
 
+extern "C" size_t zg_model_prefill_rows(const zg_model* m) { return m ? m->pf_cap : 0; }
+
+extern "C" zg_status zg_model_test_prefill_fit(zg_model* m, size_t rows) {
+  if (!m) return ZG_ERR_INVALID_ARG;
+  m->pf_fit = rows;
+  return ZG_OK;
+}
+
 extern "C" zg_status zg_model_step_waiters(const zg_model* m, uint32_t pos, uint32_t* waiters, uint32_t* slots) {
   if (!m || !waiters || !slots || pos >= m->d.max_ctx) return ZG_ERR_INVALID_ARG;
   hipSetDevice(m->ctx->device);
@@ -2094,7 +2137,7 @@ extern "C" zg_status zg_model_generate_ex(zg_model* m, const uint32_t* prompt, s
   };
   if (batched && !m->pf_ok)
     return set_error(ctx, ZG_ERR_UNSUPPORTED_QUANT, "generate: the batched prefill's GEMMs take Q4_0 / Q8_0 and plain Q4_K / Q6_K projections");
-  if (batched && (s = prefill_alloc(m))) return s;
+  if (batched && (s = prefill_alloc(m, n_prompt))) return s;
   note_rows(m, 0, prompt, n_prompt, batched ? kRowBatched : kRowDecode);
   if ((s = set_state(m, prompt[0], batched ? (uint32_t)n_prompt - 1 : 0, (uint32_t)n_prompt, (uint32_t)n_gen)))
     return s;
