@@ -28,7 +28,10 @@ def test_host_call_equals_device_call(ctx, rows, k):
             out = np.empty(rows, np.float32)
             ctx.linear_dispatch(x, w, out, k, rows, Q4_0)
             assert np.array_equal(out.view(np.uint32), want)
-        for s, e in {(0, 1), (rows - 1, rows), (min(3, rows - 1), rows), (rows // 2, rows // 2)}:
+        # starts at every offset in a 16-byte piece, and ends around the staging's
+        # limit of 16,384 rows counted from the piece that holds the start
+        ends = {(min(1, rows - 1), min(e, rows)) for e in (16381, 16382, 16383, 16384)}
+        for s, e in ends | {(0, 1), (rows - 1, rows), (min(2, rows - 1), rows), (min(3, rows - 1), rows), (rows // 2, rows // 2)}:
             out = np.full(rows, -7.0, np.float32)
             ctx.linear_range(x, w, out, k, rows, Q4_0, s, e)
             assert np.array_equal(out[s:e].view(np.uint32), want[s:e]) and np.all(out[:s] == -7.0) and np.all(out[e:] == -7.0)

@@ -737,12 +737,14 @@ zg_status zg::stage_in(zg_ctx* ctx, const void* src, size_t bytes, DevBuf& dst) 
 zg_status zg::fetch_out(zg_ctx* ctx, const void* src, const HostOut* out, size_t n) {
   size_t total = 0;
   for (size_t i = 0; i < n; i++) total += out[i].bytes;
-  const bool staged = ctx->h_pinned && total <= kStageOut && total % 4 == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0;
+  // (staged copies start at the 16-byte piece that src lies in)
+  const size_t lead = reinterpret_cast<uintptr_t>(src) & 15;
+  const bool staged = ctx->h_pinned && total + lead <= kStageOut && total % 4 == 0 && lead % 4 == 0;
   uint8_t* pin = static_cast<uint8_t*>(ctx->h_pinned) + kStageIn;
   zg_status s = ZG_OK;
   if (staged) {
     ctx->stage_busy = true;
-    s = hip_check(ctx, stage_copy(src, pin, total, ctx->stream), "download");
+    s = hip_check(ctx, stage_copy(static_cast<const uint8_t*>(src) - lead, pin, lead + total, ctx->stream), "download");
   } else {
     size_t off = 0;
     for (size_t i = 0; i < n && !s; off += out[i].bytes, i++)
@@ -754,7 +756,7 @@ zg_status zg::fetch_out(zg_ctx* ctx, const void* src, const HostOut* out, size_t
   if ((s = hip_check(ctx, hipStreamSynchronize(ctx->stream), "sync"))) return s;
   ctx->stage_busy = false;
   if (staged)
-    for (size_t i = 0, off = 0; i < n; off += out[i].bytes, i++) memcpy(out[i].dst, pin + off, out[i].bytes);
+    for (size_t i = 0, off = lead; i < n; off += out[i].bytes, i++) memcpy(out[i].dst, pin + off, out[i].bytes);
   return ZG_OK;
 }
 
@@ -778,15 +780,8 @@ extern "C" zg_status zg_linear_range(zg_ctx* ctx, const float* x, const void* w,
   s = run_linear(ctx, static_cast<const float*>(ctx->d_x.ptr), dw, dout, in_dim, out_dim, ggml_type, il, start, end,
                  EPI_STORE, nullptr, nullptr, PRO_PLAIN, nullptr, 0.0f, ctx->stream);
   if (s) return s;
-  // (from a 16-byte aligned row on, so that a small range takes the staged copy)
-  const size_t lead = start % 4, at = start - lead;
-  if (lead == 0 || end == start) {
-    const HostOut o{out + start, (end - start) * sizeof(float)};
-    return fetch_out(ctx, dout + start, &o, 1);
-  }
-  float skip[4];
-  const HostOut o[2] = {{skip, lead * sizeof(float)}, {out + start, (end - start) * sizeof(float)}};
-  return fetch_out(ctx, dout + at, o, 2);
+  const HostOut o{out + start, (end - start) * sizeof(float)};
+  return fetch_out(ctx, dout + start, &o, 1);
 }
 
 extern "C" zg_status zg_linear(zg_ctx* ctx, const float* x, const void* w, float* out, size_t in_dim, size_t out_dim,

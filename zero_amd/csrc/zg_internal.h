@@ -113,8 +113,9 @@ zg_status run_fused(zg_ctx* ctx, const float* x, const FusedDev* segs, size_t ns
 zg_status run_attn_o(zg_ctx* ctx, const float* part_o, const float* part_ml, int nsplit, int hd, const uint8_t* w,
                      float* y, size_t k, size_t n, uint32_t qt, uint32_t il, hipStream_t st);
 zg_status stage_in(zg_ctx* ctx, const void* src, size_t bytes, DevBuf& dst);
-// Copies of n <= 3 pieces of device results to host memory, `src` holding
-// them back to back, and the wait for the stream (a host call's last step).
+// Copies of n <= 3 pieces of device results to host memory, `src` (anywhere in
+// an allocation that starts 16-byte aligned) holding them back to back, and the
+// wait for the stream (a host call's last step).
 struct HostOut {
   void* dst;
   size_t bytes;
