@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+import zero_amd
 from zero_amd import synth
 
 pytestmark = pytest.mark.gpu
@@ -54,3 +55,26 @@ def test_host_fused_call_with_odd_segments(ctx):
         assert all(np.array_equal(a.view(np.uint32), b.view(np.uint32)) for a, b in zip(one, outs))
     finally:
         ctx.clear()
+
+
+def test_staging_begins_with_the_second_host_call(ctx):
+    """A fresh context: device calls, then host calls on changing activations,
+    with outputs that fit the staging and one that does not; each gives the
+    device call's bits, so nothing of an earlier call's bytes is read again."""
+    rng = np.random.default_rng(11)
+    k = 64
+    own = zero_amd.Context(0)
+    try:
+        for rows in (8, 16388, 12):
+            w = synth.weight(rng, Q4_0, rows, k, 1)
+            wd = torch.from_numpy(w).cuda()
+            own.register(w, Q4_0, 1)
+            for _ in range(4):
+                x = synth.activations(rng, k)
+                y = torch.empty(rows, dtype=torch.float32, device="cuda")
+                own.linear_dev(torch.from_numpy(x).cuda(), wd, y, k, rows, Q4_0, 1)
+                out = np.empty(rows, np.float32)
+                own.linear_dispatch(x, w, out, k, rows, Q4_0)
+                assert np.array_equal(out.view(np.uint32), y.cpu().numpy().view(np.uint32))
+    finally:
+        own.close()

@@ -110,14 +110,8 @@ extern "C" zg_status zg_init(int device, zg_ctx** out) {
     delete ctx;
     return ZG_ERR_OUT_OF_MEMORY;
   }
-  // without it the host-pointer calls copy pageable memory
-  if (hipHostMalloc(&ctx->h_pinned, kStageIn + kStageOut, hipHostMallocDefault) != hipSuccess) {
-    (void)hipGetLastError();
-    ctx->h_pinned = nullptr;
-  }
   // the no-allocation entry point's scratch address on this device
   if (noalloc_scratch_setup(ctx) != ZG_OK) {
-    if (ctx->h_pinned) hipHostFree(ctx->h_pinned);
     hipFree(ctx->d_best);
     hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -712,10 +706,24 @@ static hipError_t stage_copy(const void* src, void* dst, size_t bytes, hipStream
   return hipGetLastError();
 }
 
-// The pinned staging memory, free of an earlier call's copies (a call that
-// failed before its wait); false when there is none.
+// The context's pinned staging memory, allocated by its second host call: the
+// allocation takes 62 us, what five calls gain, and zg_init and a single call
+// are not for that.  False when there is none yet or none could be had: the
+// call then copies pageable memory.
+static bool stage_have(zg_ctx* ctx) {
+  if (!ctx->h_pinned && ctx->host_calls > 1 && !ctx->no_pinned &&
+      hipHostMalloc(&ctx->h_pinned, kStageIn + kStageOut, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    ctx->h_pinned = nullptr;
+    ctx->no_pinned = true;
+  }
+  return ctx->h_pinned != nullptr;
+}
+
+// The same, free of an earlier call's copies (a call that failed before its
+// wait).
 static bool stage_ready(zg_ctx* ctx) {
-  if (!ctx->h_pinned) return false;
+  if (!stage_have(ctx)) return false;
   if (ctx->stage_busy) {
     if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
     ctx->stage_busy = false;
@@ -724,6 +732,7 @@ static bool stage_ready(zg_ctx* ctx) {
 }
 
 zg_status zg::stage_in(zg_ctx* ctx, const void* src, size_t bytes, DevBuf& dst) {
+  if (ctx->host_calls < 2) ctx->host_calls++;
   zg_status s = ensure_buf(ctx, dst, bytes);
   if (s) return s;
   if (bytes <= kStageIn && bytes % 4 == 0 && stage_ready(ctx)) {
@@ -739,7 +748,7 @@ zg_status zg::fetch_out(zg_ctx* ctx, const void* src, const HostOut* out, size_t
   for (size_t i = 0; i < n; i++) total += out[i].bytes;
   // (staged copies start at the 16-byte piece that src lies in)
   const size_t lead = reinterpret_cast<uintptr_t>(src) & 15;
-  const bool staged = ctx->h_pinned && total + lead <= kStageOut && total % 4 == 0 && lead % 4 == 0;
+  const bool staged = total + lead <= kStageOut && total % 4 == 0 && lead % 4 == 0 && stage_have(ctx);
   uint8_t* pin = static_cast<uint8_t*>(ctx->h_pinned) + kStageIn;
   zg_status s = ZG_OK;
   if (staged) {

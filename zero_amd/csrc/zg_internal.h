@@ -64,9 +64,12 @@ struct zg_ctx {
   std::vector<zg::RegEntry> reg;  // sorted by key
   zg::DevBuf d_x, d_out, d_aux;
   // pinned staging of the host-pointer calls: kStageIn bytes in, then
-  // kStageOut bytes out (null: none could be had).  stage_busy: a copy kernel
-  // on the stream may still read or write it (cleared by the call's sync).
+  // kStageOut bytes out (null: not allocated; no_pinned: none could be had;
+  // host_calls: 0, 1 or more such calls so far).  stage_busy: a copy kernel on the stream may still read or write it
+  // (cleared by the call's sync).
   void* h_pinned = nullptr;
+  bool no_pinned = false;
+  uint8_t host_calls = 0;
   bool stage_busy = false;
   uint64_t* d_best = nullptr;
   std::string last_error;
