@@ -334,6 +334,20 @@ zg_status zg_model_test_drop_qkv_stores(zg_model *m, int32_t layer);
  * waiting workgroups of all launches in flight are fewer than the slots. */
 zg_status zg_model_step_waiters(const zg_model *m, uint32_t pos, uint32_t *waiters, uint32_t *slots);
 
+/* The batched prefill's causal attention on its own (device pointers, 16-byte
+ * aligned, asynchronous on `stream`, NULL the context's): row z of n sits at
+ * position pos0 + z; its query heads d_q [n][n_q * head_dim] are normalised
+ * and rotated already and attend to cache rows 0..pos0 + z of d_k and d_v
+ * [rows][n_kv * head_dim].  The caches hold pos0 + n rows rounded up to a
+ * multiple of 16; the rows past the last position are read and do not enter
+ * the result.  Scores are scaled by 1 / sqrt(head_dim).  Rows go to d_out
+ * (fp32) when it is given, else Q8_0-encoded to d_qs (int8) and d_d (fp16
+ * bits per 32 values).  A max score or exp-sum that is not finite sets bit 2
+ * of *d_err.  head_dim 64 or 128, up to 8 query heads per KV head. */
+zg_status zg_prefill_attention_dev(zg_ctx *ctx, const float *d_q, const float *d_k, const float *d_v, float *d_out,
+                                   int8_t *d_qs, uint16_t *d_d, uint32_t *d_err, uint32_t n_q, uint32_t n_kv,
+                                   uint32_t head_dim, size_t n, uint32_t pos0, void *stream);
+
 /* Rows that the batched prefill's buffers hold now (0 before its first call):
  * the longest prompt so far in steps of 512, at most 2048 and max_ctx; fewer
  * where that did not fit in device memory, down to 512.  Longer prompts run

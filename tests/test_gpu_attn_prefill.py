@@ -5,10 +5,11 @@ tiles: 16-key tiles, 32 query columns (16 rows of two heads of a KV head, or
 A row's bits depend on its own position and keys only, so any split of a
 prompt into calls gives the same final rows bit for bit; against the oracle
 (fp32 attention in its own order) the prefill differs by single roundings of
-the 8-bit activations.
+the 8-bit activations.  The attention on its own is compared with float64.
 """
 import numpy as np
 import pytest
+import torch
 
 from zero_amd import _lib, synth
 from zero_amd.model import GpuModel
@@ -38,8 +39,9 @@ def test_prefill_attention_tile_edges(ctx, zo, n_q, n_kv, hd, o_kq):
             tok, mx, hid = gm.prefill(prompt[:n], want_hidden=True)
             ref = om.prefill_q8(prompt[:n])
             # the roundings of 8-bit activations that another summation order
-            # flips move a tiny model's hidden state by up to 5e-3 each; an
-            # attention mistake by the size of the state
+            # flips move a tiny model's hidden state by up to 5e-3 each: this
+            # bar sees a wrong layout or row, not a single key (those are
+            # pinned against float64 below)
             assert np.max(np.abs(hid - ref)) / np.max(np.abs(ref)) <= 2e-2, n
             for cut in {1, 7, 16, n // 2, n - 1}:
                 if 0 < cut < n:
@@ -132,3 +134,89 @@ def test_prefill_row_buffers_follow_the_prompt_and_the_memory(ctx):
     finally:
         gm.close()
         ctx.clear()
+
+
+def attention(ctx, q, k, v, n_q, n_kv, hd, pos0, q8=False):
+    """zg_prefill_attention_dev on host arrays: rows, or (int8, scale) rows."""
+    n, ctx_rows = q.shape[0], pos0 + q.shape[0]
+    pad = lambda a: np.concatenate([a, np.full((-ctx_rows % 16, n_kv * hd), np.nan, np.float32)])  # noqa: E731
+    qd, kd, vd = (torch.from_numpy(a).cuda() for a in (q, pad(k), pad(v)))
+    out = torch.full((n + 1, n_q * hd), -7.0, dtype=torch.float32, device="cuda")
+    qs = torch.full((n + 1, n_q * hd), 77, dtype=torch.int8, device="cuda")
+    d = torch.full((n + 1, n_q * hd // 32), -1, dtype=torch.int16, device="cuda")
+    err = torch.zeros(1, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    ctx.check(ctx.lib.zg_prefill_attention_dev(ctx.h, qd.data_ptr(), kd.data_ptr(), vd.data_ptr(),
+                                               None if q8 else out.data_ptr(), qs.data_ptr(), d.data_ptr(), err.data_ptr(),
+                                               n_q, n_kv, hd, n, pos0, None))
+    torch.cuda.synchronize()
+    out, qs, d = out.cpu().numpy(), qs.cpu().numpy(), d.cpu().numpy()
+    # nothing past the last row, and only the asked-for form
+    assert np.all(out[n if not q8 else 0:] == -7.0) and np.all(qs[n if q8 else 0:] == 77) and np.all(d[n if q8 else 0:] == -1)
+    return (qs[:n], d[:n].view(np.float16), int(err)) if q8 else (out[:n], int(err))
+
+
+def attention_f64(q, k, v, n_q, n_kv, hd, pos0):
+    n, g = q.shape[0], n_q // n_kv
+    q, k, v = (a.astype(np.float64) for a in (q, k, v))
+    out = np.empty((n, n_q * hd))
+    seen = np.arange(pos0 + n)[None] <= pos0 + np.arange(n)[:, None]
+    for h in range(n_q):
+        kv = slice(h // g * hd, (h // g + 1) * hd)
+        s = q[:, h * hd:(h + 1) * hd] @ k[:, kv].T / np.sqrt(hd)
+        s = np.where(seen, s, -np.inf)
+        p = np.exp(s - s.max(1, keepdims=True))
+        out[:, h * hd:(h + 1) * hd] = p / p.sum(1, keepdims=True) @ v[:, kv]
+    return out
+
+
+# query heads per KV head 1, 2, 3 and 8, both head dims; contexts of one tile,
+# four (the short form's most), five, a tile edge and a row either side, more
+# than one round of the eight waves, at the start of the cache and behind rows
+@pytest.mark.parametrize("n,pos0", [(1, 0), (16, 0), (17, 0), (64, 0), (65, 0), (127, 0), (128, 0), (129, 0), (257, 0),
+                                    (1, 63), (1, 64), (15, 17), (33, 128), (40, 250)])
+@pytest.mark.parametrize("n_q,n_kv,hd", [(2, 2, 128), (4, 2, 64), (4, 2, 128), (6, 2, 64), (3, 1, 128), (8, 1, 64)])
+def test_attention_against_float64(ctx, n_q, n_kv, hd, n, pos0):
+    """Scores of spread about 1, values of spread 1: an fp32 score is off by at
+    most hd * 2^-24 * sum |q k| / sqrt(hd) (under 1e-5 here, most of it far
+    below), which moves the weights by as much relatively and the row by 1e-5
+    of the largest value.  A key dropped, doubled or let past the mask moves
+    it by its weight, 1 / 290 and more."""
+    rng = np.random.default_rng(n + 7 * pos0 + 100 * n_q + hd)
+    rows = pos0 + n
+    q = rng.standard_normal((n, n_q * hd)).astype(np.float32)
+    k, v = (rng.standard_normal((rows, n_kv * hd)).astype(np.float32) for _ in range(2))
+    want = attention_f64(q, k, v, n_q, n_kv, hd, pos0)
+    got, err = attention(ctx, q, k, v, n_q, n_kv, hd, pos0)
+    assert err == 0 and np.max(np.abs(got - want)) <= 1e-5 * np.max(np.abs(v))
+    qs, d, err = attention(ctx, q, k, v, n_q, n_kv, hd, pos0, q8=True)
+    # a block's scale is max / 127 rounded to fp16 (2^-11), its values rounded
+    # to half a step and clipped at 127 of them
+    b, dd = want.reshape(n, -1, 32), d.astype(np.float64)[..., None]
+    step = np.max(np.abs(b), 2, keepdims=True) / 127
+    assert err == 0 and np.all(np.abs(dd - step) <= step * 2.0 ** -10)
+    assert np.all(np.abs(qs.reshape(b.shape) * step - b) <= step * 0.5 + 1e-5 * np.max(np.abs(v)))
+
+
+@pytest.mark.parametrize("n_q,n_kv,hd,n,pos0", [(2, 2, 128, 150, 0), (4, 2, 64, 40, 100), (3, 1, 64, 60, 0)])
+def test_attention_single_keys(ctx, n_q, n_kv, hd, n, pos0):
+    """Every row's query picks one key (the first, its own, tile edges, ...),
+    whose score is far above the others': the row is that key's value row."""
+    rng = np.random.default_rng(hd + n)
+    rows, g = pos0 + n, n_q // n_kv
+    k = rng.choice([-1.0, 1.0], size=(rows, n_kv * hd)).astype(np.float32)
+    v = rng.standard_normal((rows, n_kv * hd)).astype(np.float32)
+    pick = np.empty((n, n_q), np.int64)
+    q = np.empty((n, n_q * hd), np.float32)
+    for z in range(n):
+        p = pos0 + z
+        edges = [c for c in (0, p, p - 1, p // 16 * 16, p // 16 * 16 - 1, p // 128 * 128, p // 2) if c >= 0]
+        for h in range(n_q):
+            pick[z, h] = edges[(z + h) % len(edges)]
+            q[z, h * hd:(h + 1) * hd] = 8 * k[pick[z, h], h // g * hd:(h // g + 1) * hd]
+    got, err = attention(ctx, q, k, v, n_q, n_kv, hd, pos0)
+    # the picked score is 8 sqrt(hd) and another's below 0.7 of it (keys of
+    # random signs): their weights are under exp(-19) each
+    for h in range(n_q):
+        want = v[pick[:, h], h // g * hd:(h // g + 1) * hd]
+        assert err == 0 and np.max(np.abs(got[:, h * hd:(h + 1) * hd] - want)) <= 1e-5, h

@@ -2017,6 +2017,24 @@ extern "C" zg_status zg_model_test_drop_qkv_stores(zg_model* m, int32_t layer) {
   return s;
 }
 
+extern "C" zg_status zg_prefill_attention_dev(zg_ctx* ctx, const float* d_q, const float* d_k, const float* d_v, float* d_out,
+                                              int8_t* d_qs, uint16_t* d_d, uint32_t* d_err, uint32_t n_q, uint32_t n_kv,
+                                              uint32_t head_dim, size_t n, uint32_t pos0, void* stream) {
+  if (!ctx) return ZG_ERR_INVALID_ARG;
+  if (!d_q || !d_k || !d_v || !d_err || (!d_out && !(d_qs && d_d)))
+    return set_error(ctx, ZG_ERR_INVALID_ARG, "prefill attention: null pointer");
+  if ((head_dim != 64 && head_dim != 128) || n_kv == 0 || n_kv > 256 || n_q == 0 || n_q % n_kv ||
+      n_q / n_kv > (uint32_t)kMaxG || n > 65535 || pos0 > (1u << 24))
+    return set_error(ctx, ZG_ERR_INVALID_ARG, "prefill attention: unsupported dimensions");
+  for (const void* p : {(const void*)d_q, (const void*)d_k, (const void*)d_v, (const void*)d_out, (const void*)d_qs})
+    if (reinterpret_cast<uintptr_t>(p) % 16) return set_error(ctx, ZG_ERR_INVALID_ARG, "prefill attention: misaligned pointer");
+  hipSetDevice(ctx->device);
+  const PrefillAttnArgs a{d_q, d_k, d_v, d_out, d_qs, d_d, d_err, (int)n_q, (int)n_kv, (int)n, (int)pos0,
+                          1.0f / sqrtf((float)head_dim)};
+  return hip_check(ctx, launch_attn_prefill(a, (int)head_dim, stream ? static_cast<hipStream_t>(stream) : ctx->stream),
+                   "prefill attention launch");
+}
+
 extern "C" size_t zg_model_prefill_rows(const zg_model* m) { return m ? m->pf_cap : 0; }
 
 extern "C" zg_status zg_model_test_prefill_fit(zg_model* m, size_t rows) {
