@@ -53,6 +53,24 @@ def test_q8act_scales_by_mfma(ctx, zo, wt, il, m, n):
     check_q8act(ctx, zo, w, x, wt, il, m, n, k)
 
 
+# the same kernel on split-scale groups (in_dims a multiple of 512), as a
+# model's long prefill runs it: whole tiles, and partial ones in both directions
+@pytest.mark.parametrize("wt", [Q4_0, Q8_0])
+@pytest.mark.parametrize("m,n", [(64, 49152), (65, 24644)])
+def test_q8act_scales_by_mfma_split_groups(ctx, wt, m, n):
+    k = 512
+    rng = np.random.default_rng(m + n + wt)
+    w = synth.weight(rng, wt, n, k, 4)
+    qs = torch.empty((m, k), dtype=torch.int8, device="cuda")
+    d = torch.empty((m, k // 32), dtype=torch.int16, device="cuda")
+    ctx.quantize_q8_0_split_dev(dev(synth.activations(rng, m * k).reshape(m, k)), qs, d, m, k)
+    ys = []
+    for il, wb in ((4, w), (5, synth.x4_split(w, n, k, wt))):
+        ys.append(torch.full((m, n), -3.0, dtype=torch.float32, device="cuda"))
+        ctx.gemm_q8act_dev(qs, d, dev(wb), ys[-1], m, n, k, wt, il)
+    assert same_bits(ys[0].cpu().numpy(), ys[1].cpu().numpy())
+
+
 def check_q8act(ctx, zo, w, x, wt, il, m, n, k):
     qs = torch.empty((m, k), dtype=torch.int8, device="cuda")
     d = torch.empty((m, k // 32), dtype=torch.int16, device="cuda")

@@ -40,6 +40,30 @@ def test_decode_across_the_long_context_switch(ctx, zo, hidden, lin, n_q, n_kv, 
         ctx.clear()
 
 
+# the fused long form's second round of 128 rows: eight splits hold 128 rows
+# each at position 1,023 and 136 from 1,024 on
+@pytest.mark.parametrize("lin,n_q,n_kv,hd", [((synth.Q4_0, 4), 8, 4, 128), ((synth.Q4K, 1), 4, 2, 64)])
+def test_decode_across_the_second_round(ctx, zo, lin, n_q, n_kv, hd):
+    cfg = synth.ModelConfig(n_layers=1, hidden=2048, ffn=512, n_q_heads=n_q, n_kv_heads=n_kv, head_dim=hd, vocab_padded=512,
+                            vocab_real=500, max_ctx=1100, lin_type=lin[0], lin_interleave=lin[1])
+    model = synth.random_model(cfg, seed=3 * hd)
+    gm, om = GpuModel(ctx, model), zo.OracleModel(model)
+    try:
+        prompt = synth.prompt(hd + 1, 1016, cfg.vocab_real)
+        toks, _, _ = gm.generate(prompt, 80)
+        assert np.array_equal(toks, om.generate(prompt, 80))
+        for pos in list(range(1020, 1030)) + [1060, 1094]:
+            t = int(toks[pos - 1016])
+            nxt, _, hid, _ = gm.step(t, pos, want_hidden=True)
+            assert nxt == int(toks[pos - 1015])
+            ref = om.forward(t, pos)
+            assert np.max(np.abs(hid - ref)) / np.max(np.abs(ref)) <= REL_TOL
+    finally:
+        gm.close()
+        om.close()
+        ctx.clear()
+
+
 # (query heads, KV heads, head dim): splits of the steps past the switch
 @pytest.mark.parametrize("n_q,n_kv,hd,splits", [(16, 8, 128, 8), (22, 11, 128, 8), (24, 8, 128, 6), (32, 8, 128, 6),
                                                 (31, 31, 64, 8), (32, 8, 64, 6)])

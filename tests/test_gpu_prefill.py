@@ -233,18 +233,23 @@ def test_prefill_chunks_bit_identical(ctx, tiny):
         ctx.clear()
 
 
-def test_prefill_longer_than_a_chunk(ctx, zo):
-    """620 rows: one 512-row chunk, then 108 rows attending to it."""
+# one 2,048-row chunk, then 12 rows attending to it; and the chunks of 512 rows
+# that a model takes whose larger row buffers do not fit
+@pytest.mark.parametrize("n,fit", [(2060, 0), (620, 512)])
+def test_prefill_longer_than_a_chunk(ctx, zo, n, fit):
     cfg = synth.ModelConfig(n_layers=1, hidden=128, ffn=256, n_q_heads=2, n_kv_heads=1, head_dim=64,
-                            vocab_padded=512, vocab_real=500, max_ctx=640)
+                            vocab_padded=512, vocab_real=500, max_ctx=n + 20)
     model = synth.random_model(cfg, seed=9)
     gm = GpuModel(ctx, model)
     om = zo.OracleModel(model)
     try:
-        prompt = synth.prompt(41, 620, cfg.vocab_real)
+        prompt = synth.prompt(41, n, cfg.vocab_real)
+        assert ctx.lib.zg_model_test_prefill_fit(gm.h, fit) == _lib.ZG_OK
         tok, _, hid = gm.prefill(prompt, want_hidden=True)
+        assert ctx.lib.zg_model_prefill_rows(gm.h) == (fit or 2048)  # fewer than the prompt's
         h_ref = om.prefill_q8(prompt)
         rc, t_ref, _, _ = om.lm_head()
+        print(f"n={n}: hidden rel err {rel_err(hid, h_ref):.2e}")
         assert rel_err(hid, h_ref) <= REL_TOL and tok == t_ref
     finally:
         om.close()
@@ -427,21 +432,25 @@ def test_qwen3_1_7b_shape_q4_k_m_batched_prefill_matches_oracle(ctx, zo):
         ctx.clear()
 
 
-def test_k_quant_prefill_longer_than_a_chunk(ctx, zo):
-    """620 rows of a Q4_K / Q6_K model (hidden 256: whole superblocks): one
-    512-row chunk of Q8_K GEMMs, then 108 rows attending to its cache rows."""
+@pytest.mark.parametrize("n,fit", [(2060, 0), (620, 512)])
+def test_k_quant_prefill_longer_than_a_chunk(ctx, zo, n, fit):
+    """A Q4_K / Q6_K model (hidden 256: whole superblocks): chunks of Q8_K
+    GEMMs, the second attending to the first's cache rows."""
     cfg = synth.ModelConfig(n_layers=2, hidden=256, ffn=512, n_q_heads=4, n_kv_heads=2, head_dim=64,
-                            vocab_padded=512, vocab_real=500, max_ctx=640, embd_type=synth.Q4K,
+                            vocab_padded=512, vocab_real=500, max_ctx=n + 20, embd_type=synth.Q4K,
                             head_type=synth.Q6K, head_interleave=1, layer_quants=synth.q4_k_m_layers(2))
     model = synth.random_model(cfg, seed=19)
     gm = GpuModel(ctx, model)
     om = zo.OracleModel(model)
     try:
-        prompt = synth.prompt(43, 620, cfg.vocab_real)
+        prompt = synth.prompt(43, n, cfg.vocab_real)
+        assert ctx.lib.zg_model_test_prefill_fit(gm.h, fit) == _lib.ZG_OK
         tok, _, hid = gm.prefill(prompt, want_hidden=True)
+        assert ctx.lib.zg_model_prefill_rows(gm.h) == (fit or 2048)
         h_ref = om.prefill_q8(prompt)
         rc, t_ref, _, _ = om.lm_head()
         assert rc == 0
+        print(f"n={n}: hidden rel err {rel_err(hid, h_ref):.2e}")
         assert rel_err(hid, h_ref) <= REL_TOL and tok == t_ref
     finally:
         om.close()
