@@ -527,9 +527,25 @@ def _profile_workloads(ctx, names, reps: int):
             y = torch.empty(rows, device="cuda")
             run(name, lambda i: ctx.linear_dev(x, wd[i], y, k, rows, qt, 1), len(wd))
             del wd
-        elif name in ("gemm_up", "gemm_down"):
-            M = 512
-            n_out, k = (6144, 2048) if name == "gemm_up" else (2048, 6144)
+        elif name in ("wide_q4", "wide_q8"):  # an in_dim outside the strip kernel's range, plain rows
+            qt, rows, k = (synth.Q4_0 if name == "wide_q4" else synth.Q8_0), 4096, 11_008
+            wd = rotating(synth.weight(rng, qt, rows, k, 1))
+            y = torch.empty(rows, device="cuda")
+            run(name, lambda i: ctx.linear_dev(x, wd[i], y, k, rows, qt, 1), len(wd))
+            del wd
+        elif name == "prefill_attn":  # one layer's attention of 1,800 prompt rows, Q8_0 rows out
+            n, nq, nkv, hd = 1800, 16, 8, 128
+            q = torch.randn(n, nq * hd, device="cuda")
+            kc, vc = (torch.randn((n + 15) // 16 * 16, nkv * hd, device="cuda") for _ in range(2))
+            qs = torch.empty((n, nq * hd), dtype=torch.int8, device="cuda")
+            dd = torch.empty((n, nq * hd // 32), dtype=torch.int16, device="cuda")
+            err = torch.zeros(1, dtype=torch.int32, device="cuda")
+            run(name, lambda i: ctx.check(ctx.lib.zg_prefill_attention_dev(
+                ctx.h, q.data_ptr(), kc.data_ptr(), vc.data_ptr(), None, qs.data_ptr(), dd.data_ptr(), err.data_ptr(),
+                nq, nkv, hd, n, 0, None)), 1)
+        elif name in ("gemm_up", "gemm_down", "gemm_long", "gemm_few"):
+            M, n_out, k = {"gemm_up": (512, 6144, 2048), "gemm_down": (512, 2048, 6144),
+                           "gemm_long": (1800, 12_288, 2048), "gemm_few": (128, 2048, 6144)}[name]
             wd = torch.from_numpy(synth.weight(rng, synth.Q4_0, n_out, k, 4)).cuda()
             xm = torch.from_numpy(synth.activations(rng, M, k)).cuda()
             qs = torch.empty((M, k), dtype=torch.int8, device="cuda")
@@ -537,9 +553,10 @@ def _profile_workloads(ctx, names, reps: int):
             ym = torch.empty((M, n_out), device="cuda")
             ctx.quantize_q8_0_split_dev(xm, qs, dd, M, k)
             run(name, lambda i: ctx.gemm_q8act_dev(qs, dd, wd, ym, M, n_out, k, synth.Q4_0, 4), 1)
-        elif name in ("kgemm_up", "kgemm_down"):
-            M = 512
-            qt, n_out, k = (synth.Q4K, 6144, 2048) if name == "kgemm_up" else (synth.Q6K, 2048, 6144)
+        elif name in ("kgemm_up", "kgemm_down", "kgemm_300", "kgemm_few_o", "kgemm_few_down"):
+            M, qt, n_out, k = {"kgemm_up": (512, synth.Q4K, 6144, 2048), "kgemm_down": (512, synth.Q6K, 2048, 6144),
+                               "kgemm_300": (300, synth.Q4K, 6144, 2048), "kgemm_few_o": (150, synth.Q4K, 2048, 2048),
+                               "kgemm_few_down": (150, synth.Q6K, 2048, 6144)}[name]
             wd = torch.from_numpy(synth.weight(rng, qt, n_out, k, 1)).cuda()
             xm = torch.from_numpy(synth.activations(rng, M, k)).cuda()
             qs = torch.empty((M, k), dtype=torch.int8, device="cuda")
@@ -796,8 +813,9 @@ def main():
     ap.add_argument("--no-rows", action="store_true", help="skip the fused-QKV, LM-head, k-quant and GEMM lines")
     ap.add_argument("--profile", default="",
                     help="comma list of workloads to launch eagerly (no graph) for rocprofv3 counter passes, "
-                         "then exit: c1, tall, floor_c1, floor_tall, lmhead, qkv, q4k, q6k, gemm_up, gemm_down, kgemm_up, "
-                         "kgemm_down, copy")
+                         "then exit: c1, tall, floor_c1, floor_tall, lmhead, qkv, q4k, q6k, wide_q4, wide_q8, prefill_attn, "
+                         "gemm_up, gemm_down, gemm_long, gemm_few, kgemm_up, kgemm_down, kgemm_300, kgemm_few_o, "
+                         "kgemm_few_down, copy")
     ap.add_argument("--profile-reps", type=int, default=30)
     ap.add_argument("--pmc-calib", action="store_true",
                     help="first run one elementwise kernel that reads 256 MiB and writes 256 MiB, the "
