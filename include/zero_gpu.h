@@ -364,12 +364,13 @@ zg_status zg_model_test_prefill_fit(zg_model *m, size_t rows);
  * activation quantization (the packer's encoder, silicatepack.py:893-907)
  * and zg_gemm_q8act_dev-style GEMMs (Q|K|V, O, gate|up, down), with the
  * decode step's QK-norm, RoPE, causal attention and SwiGLU per row.  Writes
- * KV rows pos0..pos0+n-1 (chunks of up to 2048 rows attend to the rows
- * before them), then runs the LM head on the last row.  Leaves the model
- * ready to decode at position pos0 + n.  hidden_out (optional): the final
+ * KV rows pos0..pos0+n-1 (chunks of up to 2048 rows,
+ * zg_model_prefill_rows, attend to the rows before them), then runs the LM
+ * head on the last row.  Leaves the model ready to decode at position pos0 + n.  hidden_out (optional): the final
  * hidden state of the last row.  Activations are quantized to 8 bits, so
  * results differ from token-by-token prefill by that quantization.  The
- * GEMMs take Q4_0 / Q8_0 weights: a model with a Q4_K or Q6_K layer
+ * GEMMs take Q4_0 / Q8_0 projections, and plain Q4_K / Q6_K ones (on Q8_K
+ * rows) of widths in 64s and in_dims in 256s: a model with another layer
  * projection returns ZG_ERR_UNSUPPORTED_QUANT here (it decodes, and
  * prefills token by token). */
 zg_status zg_model_prefill(zg_model *m, const uint32_t *tokens, size_t n, uint32_t pos0,

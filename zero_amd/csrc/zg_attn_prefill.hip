@@ -28,16 +28,18 @@
 // is computed in.
 //
 // Bound: the fp32 matrix rate (32 cycles per MFMA, 128 MFMAs per tile at
-// head_dim 128; 157 TFLOP/s for the chip), then each workgroup's own prologue
-// and merge (8 us for a single short row; one workgroup fits a CU), the
-// masked half of the diagonal tiles and the last workgroups of a chunk.  K
-// and V come from L2: 16 KB per tile and wave.  16 query and 8 KV heads of 128,
-// graph replays: 512 rows at position 0 30 us, at 1024 69 us (78 TFLOP/s).
-// The form before it, one workgroup per query head and row that re-read K and
-// V for every row: prefill of 1,800 tokens 50.4 ms in all, 22.1 ms with this
-// one.  Measured and not used: 32-key tiles with v_mfma_f32_32x32x2_f32
-// (22.6 ms), V loaded a tile ahead as K is (512 rows at 1024: 74 us); without
-// the exponentials or without the loads the time hardly moves (72 and 70 us).
+// head_dim 128; 157 TFLOP/s for the chip; the matrix cores are busy 51 % of
+// the cycles of 1,800 rows), then each workgroup's own prologue and merge
+// (7.4 us for 16 rows; one workgroup fits a CU), the masked half of the
+// diagonal tiles and the last workgroups of a chunk.  K and V come from L2:
+// 16 KB per tile and wave.  16 query and 8 KV heads of 128, graph replays: 150
+// rows 15.5 us, 512 rows at position 0 28 us, at 1024 67 us (80 TFLOP/s), 1,800
+// rows 162 us.  The form before it, one workgroup per query head and row that
+// re-read K and V for every row: prefill of 1,800 tokens in 512-row chunks 50.4
+// ms in all, 22.1 ms with this one.  Measured and not used: 32-key tiles with
+// v_mfma_f32_32x32x2_f32 (22.6 ms), V loaded a tile ahead as K is (512 rows at
+// 1024: 74 us); without the exponentials or without the loads the time hardly
+// moved (72 and 70 us, of 69 then).
 #include <type_traits>
 
 #include "zg_device.h"

@@ -363,9 +363,9 @@ __device__ __forceinline__ void gemm_stage_load_full(GemmStage<WT, BM, BK, NT, B
 // product dX dW, exact in fp32 (two 11-bit significands, subnormals
 // included): one matrix instruction and two 2-byte LDS reads in place of 16
 // multiplies on the vector units, which bind the kernel, and five wider
-// reads.  The lanes that hold the other k slots read the zeros.  Graph
-// replays, Q4_0X4: 512 x 6144 x 2048 29.7 -> 26.7 us, 1800 x 12288 x 2048 172 ->
-// 149 us (608 TOPS), 1800 x 2048 x 6144 103 -> 83 us.  The 16 x 16 form keeps
+// reads.  The lanes that hold the other k slots read the zeros.  The GEMM
+// alone, graphs of 64 launches, Q4_0X4: 512 x 6144 x 2048 29.2 -> 26.4 us, 1800 x
+// 12288 x 2048 170 -> 150 us (604 TOPS), 1800 x 2048 x 6144 103 -> 83 us.  The 16 x 16 form keeps
 // its multiplies: its waves wait for latency, not for the vector units (512 x
 // 2048 x 6144 33.7 against 35.2 us).  Measured and not used: an integer bias in
 // the MFMA's C operand and a subtraction in place of the conversion (27.3 us),
