@@ -542,7 +542,7 @@ def _profile_workloads(ctx, names, reps: int):
             err = torch.zeros(1, dtype=torch.int32, device="cuda")
             run(name, lambda i: ctx.check(ctx.lib.zg_prefill_attention_dev(
                 ctx.h, q.data_ptr(), kc.data_ptr(), vc.data_ptr(), None, qs.data_ptr(), dd.data_ptr(), err.data_ptr(),
-                nq, nkv, hd, n, 0, None)), 1)
+                nq, nkv, hd, n, 0, None, 0, None)), 1)
         elif name in ("gemm_up", "gemm_down", "gemm_long", "gemm_few"):
             M, n_out, k = {"gemm_up": (512, 6144, 2048), "gemm_down": (512, 2048, 6144),
                            "gemm_long": (1800, 12_288, 2048), "gemm_few": (128, 2048, 6144)}[name]

@@ -343,10 +343,15 @@ zg_status zg_model_step_waiters(const zg_model *m, uint32_t pos, uint32_t *waite
  * the result.  Scores are scaled by 1 / sqrt(head_dim).  Rows go to d_out
  * (fp32) when it is given, else Q8_0-encoded to d_qs (int8) and d_d (fp16
  * bits per 32 values).  A max score or exp-sum that is not finite sets bit 2
- * of *d_err.  head_dim 64 or 128, up to 8 query heads per KV head. */
+ * of *d_err.  head_dim 64 or 128, up to 8 query heads per KV head.
+ * d_scratch (NULL: none): zg_prefill_attention_scratch bytes with which few
+ * rows at a long context run on more CUs, in use until the call's work on the
+ * stream is done; the results do not depend on it. */
+size_t zg_prefill_attention_scratch(uint32_t n_q, uint32_t n_kv, uint32_t head_dim, size_t n);
 zg_status zg_prefill_attention_dev(zg_ctx *ctx, const float *d_q, const float *d_k, const float *d_v, float *d_out,
                                    int8_t *d_qs, uint16_t *d_d, uint32_t *d_err, uint32_t n_q, uint32_t n_kv,
-                                   uint32_t head_dim, size_t n, uint32_t pos0, void *stream);
+                                   uint32_t head_dim, size_t n, uint32_t pos0, void *d_scratch,
+                                   size_t scratch_bytes, void *stream);
 
 /* Rows that the batched prefill's buffers hold now (0 before its first call):
  * the longest prompt so far in steps of 512, at most 2048 and max_ctx; fewer

@@ -136,7 +136,7 @@ def test_prefill_row_buffers_follow_the_prompt_and_the_memory(ctx):
         ctx.clear()
 
 
-def attention(ctx, q, k, v, n_q, n_kv, hd, pos0, q8=False):
+def attention(ctx, q, k, v, n_q, n_kv, hd, pos0, q8=False, scratch=True):
     """zg_prefill_attention_dev on host arrays: rows, or (int8, scale) rows."""
     n, ctx_rows = q.shape[0], pos0 + q.shape[0]
     pad = lambda a: np.concatenate([a, np.full((-ctx_rows % 16, n_kv * hd), np.nan, np.float32)])  # noqa: E731
@@ -145,11 +145,14 @@ def attention(ctx, q, k, v, n_q, n_kv, hd, pos0, q8=False):
     qs = torch.full((n + 1, n_q * hd), 77, dtype=torch.int8, device="cuda")
     d = torch.full((n + 1, n_q * hd // 32), -1, dtype=torch.int16, device="cuda")
     err = torch.zeros(1, dtype=torch.int32, device="cuda")
+    nb = ctx.lib.zg_prefill_attention_scratch(n_q, n_kv, hd, n) if scratch else 0
+    sc = torch.full((nb + 16,), 255, dtype=torch.uint8, device="cuda")  # NaNs, and a guard behind them
     torch.cuda.synchronize()
     ctx.check(ctx.lib.zg_prefill_attention_dev(ctx.h, qd.data_ptr(), kd.data_ptr(), vd.data_ptr(),
                                                None if q8 else out.data_ptr(), qs.data_ptr(), d.data_ptr(), err.data_ptr(),
-                                               n_q, n_kv, hd, n, pos0, None))
+                                               n_q, n_kv, hd, n, pos0, sc.data_ptr() if nb else None, nb, None))
     torch.cuda.synchronize()
+    assert torch.all(sc[nb:] == 255)
     out, qs, d = out.cpu().numpy(), qs.cpu().numpy(), d.cpu().numpy()
     # nothing past the last row, and only the asked-for form
     assert np.all(out[n if not q8 else 0:] == -7.0) and np.all(qs[n if q8 else 0:] == 77) and np.all(d[n if q8 else 0:] == -1)
@@ -174,14 +177,15 @@ def attention_f64(q, k, v, n_q, n_kv, hd, pos0):
 # four (the short form's most), five, a tile edge and a row either side, more
 # than one round of the eight waves, at the start of the cache and behind rows
 @pytest.mark.parametrize("n,pos0", [(1, 0), (16, 0), (17, 0), (64, 0), (65, 0), (127, 0), (128, 0), (129, 0), (257, 0),
-                                    (1, 63), (1, 64), (15, 17), (33, 128), (40, 250)])
+                                    (1, 63), (1, 64), (15, 17), (33, 128), (40, 250), (1, 127), (1, 128), (5, 400), (33, 300)])
 @pytest.mark.parametrize("n_q,n_kv,hd", [(2, 2, 128), (4, 2, 64), (4, 2, 128), (6, 2, 64), (3, 1, 128), (8, 1, 64)])
 def test_attention_against_float64(ctx, n_q, n_kv, hd, n, pos0):
-    """Scores of spread about 1, values of spread 1: an fp32 score is off by at
+    """With scratch (few rows behind more than four tiles share their slots
+    over workgroups) and without, the same bits.  Scores of spread about 1, values of spread 1: an fp32 score is off by at
     most hd * 2^-24 * sum |q k| / sqrt(hd) (under 1e-5 here, most of it far
     below), which moves the weights by as much relatively and the row by 1e-5
     of the largest value.  A key dropped, doubled or let past the mask moves
-    it by its weight, 1 / 290 and more."""
+    it by its weight, 1 / 405 and more."""
     rng = np.random.default_rng(n + 7 * pos0 + 100 * n_q + hd)
     rows = pos0 + n
     q = rng.standard_normal((n, n_q * hd)).astype(np.float32)
@@ -189,6 +193,8 @@ def test_attention_against_float64(ctx, n_q, n_kv, hd, n, pos0):
     want = attention_f64(q, k, v, n_q, n_kv, hd, pos0)
     got, err = attention(ctx, q, k, v, n_q, n_kv, hd, pos0)
     assert err == 0 and np.max(np.abs(got - want)) <= 1e-5 * np.max(np.abs(v))
+    one, err = attention(ctx, q, k, v, n_q, n_kv, hd, pos0, scratch=False)
+    assert err == 0 and np.array_equal(one.view(np.uint32), got.view(np.uint32))
     qs, d, err = attention(ctx, q, k, v, n_q, n_kv, hd, pos0, q8=True)
     # a block's scale is max / 127 rounded to fp16 (2^-11), its values rounded
     # to half a step and clipped at 127 of them
@@ -196,6 +202,12 @@ def test_attention_against_float64(ctx, n_q, n_kv, hd, n, pos0):
     step = np.max(np.abs(b), 2, keepdims=True) / 127
     assert err == 0 and np.all(np.abs(dd - step) <= step * 2.0 ** -10)
     assert np.all(np.abs(qs.reshape(b.shape) * step - b) <= step * 0.5 + 1e-5 * np.max(np.abs(v)))
+
+
+# more than 64 units of five to eight tiles, and of nine: the long form
+@pytest.mark.parametrize("n,pos0", [(113, 0), (128, 0), (113, 16)])
+def test_attention_of_many_units(ctx, n, pos0):
+    test_attention_against_float64(ctx, 24, 12, 64, n, pos0)
 
 
 @pytest.mark.parametrize("n_q,n_kv,hd,n,pos0", [(2, 2, 128, 150, 0), (4, 2, 64, 40, 100), (3, 1, 64, 60, 0)])

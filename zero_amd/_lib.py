@@ -149,7 +149,8 @@ SIGNATURES = {
     "zg_model_reset": (None, [_P]),
     "zg_model_first_nonfinite": (_S, [_P, C.c_char_p, _S]),
     "zg_model_test_drop_qkv_stores": (_ST, [_P, C.c_int32]),
-    "zg_prefill_attention_dev": (_ST, [_P] * 8 + [_U32, _U32, _U32, _S, _U32, _P]),
+    "zg_prefill_attention_scratch": (C.c_size_t, [_U32, _U32, _U32, _S]),
+    "zg_prefill_attention_dev": (_ST, [_P] * 8 + [_U32, _U32, _U32, _S, _U32, _P, _S, _P]),
     "zg_model_prefill_rows": (C.c_size_t, [_P]),
     "zg_model_test_prefill_fit": (_ST, [_P, C.c_size_t]),
     "zg_model_step_waiters": (_ST, [_P, C.c_uint32, C.POINTER(C.c_uint32), C.POINTER(C.c_uint32)]),

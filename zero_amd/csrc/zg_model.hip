@@ -1024,6 +1024,8 @@ struct zg_model {
   // holds them all), allocated by the first call and grown by longer prompts
   size_t pf_cap = 0;
   void* pf_mem = nullptr;
+  float* pf_part = nullptr;  // the prefill attention's scratch
+  size_t pf_part_bytes = 0;
   size_t pf_fit = 0;  // test hook: buffers of more rows do not fit (0: none)
   float *pf_x = nullptr, *pf_q = nullptr, *pf_k = nullptr, *pf_v = nullptr;
   float *pf_g = nullptr, *pf_u = nullptr;
@@ -1057,7 +1059,7 @@ enum RowKind : uint8_t { kRowUnknown = 0, kRowDecode = 1, kRowBatched = 2 };
 // Qwen3-1.7B shape, Q4_0X4 / Q4_K_M: 17.3 / 21.3 ms, against 22.2 / 29.3 ms
 // in chunks of 512 and 18.8 / 23.3 ms of 1,024); the row buffers take 83 KB a
 // row at that shape, in steps of kPrefillStep rows by the longest prompt (42
-// MB up to 512 rows, 170 MB from 1,537 on).
+// MB up to 512 rows, 170 MB from 1,537 on), and the attention's scratch 8.5 MB.
 constexpr size_t kPrefillChunk = 2048;
 constexpr size_t kPrefillStep = 512;
 
@@ -1474,6 +1476,11 @@ static size_t prefill_layout(zg_model* m, size_t C, uint8_t* base) {
   part(&m->pf_u, C * F * 4);
   part(&m->pf_qs, C * kmax);
   part(&m->pf_qd, C * (kmax / 32) * 2);
+  // the attention's scratch for few rows: the most of any row count up to C
+  m->pf_part_bytes = 0;
+  for (size_t n = 1; n <= C; n++)
+    m->pf_part_bytes = std::max(m->pf_part_bytes, attn_prefill_scratch((int)d.n_q_heads, (int)d.n_kv_heads, (int)d.head_dim, (int)n));
+  part(&m->pf_part, m->pf_part_bytes);
   if (m->pf_kq) {
     part(&m->pf_ks, C * kmax);
     part(&m->pf_k8, C * (kmax / 256) * 4);
@@ -1585,7 +1592,7 @@ static zg_status prefill_chunk(zg_model* m, const uint32_t* d_tokens, size_t n, 
     if ((s = hip_check(ctx, hipGetLastError(), "prefill qk-rope launch"))) break;
     const bool o_kq = kq_type(L.qt[ZG_PROJ_O]);
     const PrefillAttnArgs pa{m->pf_q, kc, vc, o_kq ? m->pf_a : nullptr, m->pf_qs, m->pf_qd, &m->st->err, nq, nkv, (int)n,
-                             (int)pos0, scale};
+                             (int)pos0, scale, m->pf_part, m->pf_part_bytes};
     if ((s = hip_check(ctx, launch_attn_prefill(pa, HD, st), "prefill attention launch"))) break;
     if (o_kq && (s = run_quantize_q8k_split(ctx, m->pf_a, m->pf_ks, m->pf_k8, m->pf_kb, n, qd, st))) break;
     const GemmSegDev o{L.o, m->pf_x, (size_t)H};
@@ -2017,20 +2024,29 @@ extern "C" zg_status zg_model_test_drop_qkv_stores(zg_model* m, int32_t layer) {
   return s;
 }
 
+extern "C" size_t zg_prefill_attention_scratch(uint32_t n_q, uint32_t n_kv, uint32_t head_dim, size_t n) {
+  if (n_kv == 0 || n_kv > 256 || n_q == 0 || n_q % n_kv || n_q / n_kv > (uint32_t)kMaxG || n > 65535 ||
+      (head_dim != 64 && head_dim != 128))
+    return 0;
+  return attn_prefill_scratch((int)n_q, (int)n_kv, (int)head_dim, (int)n);
+}
+
 extern "C" zg_status zg_prefill_attention_dev(zg_ctx* ctx, const float* d_q, const float* d_k, const float* d_v, float* d_out,
                                               int8_t* d_qs, uint16_t* d_d, uint32_t* d_err, uint32_t n_q, uint32_t n_kv,
-                                              uint32_t head_dim, size_t n, uint32_t pos0, void* stream) {
+                                              uint32_t head_dim, size_t n, uint32_t pos0, void* d_scratch,
+                                              size_t scratch_bytes, void* stream) {
   if (!ctx) return ZG_ERR_INVALID_ARG;
   if (!d_q || !d_k || !d_v || !d_err || (!d_out && !(d_qs && d_d)))
     return set_error(ctx, ZG_ERR_INVALID_ARG, "prefill attention: null pointer");
   if ((head_dim != 64 && head_dim != 128) || n_kv == 0 || n_kv > 256 || n_q == 0 || n_q % n_kv ||
       n_q / n_kv > (uint32_t)kMaxG || n > 65535 || pos0 > (1u << 24))
     return set_error(ctx, ZG_ERR_INVALID_ARG, "prefill attention: unsupported dimensions");
-  for (const void* p : {(const void*)d_q, (const void*)d_k, (const void*)d_v, (const void*)d_out, (const void*)d_qs})
+  for (const void* p : {(const void*)d_q, (const void*)d_k, (const void*)d_v, (const void*)d_out, (const void*)d_qs,
+                        (const void*)d_scratch})
     if (reinterpret_cast<uintptr_t>(p) % 16) return set_error(ctx, ZG_ERR_INVALID_ARG, "prefill attention: misaligned pointer");
   hipSetDevice(ctx->device);
   const PrefillAttnArgs a{d_q, d_k, d_v, d_out, d_qs, d_d, d_err, (int)n_q, (int)n_kv, (int)n, (int)pos0,
-                          1.0f / sqrtf((float)head_dim)};
+                          1.0f / sqrtf((float)head_dim), static_cast<float*>(d_scratch), d_scratch ? scratch_bytes : 0};
   return hip_check(ctx, launch_attn_prefill(a, (int)head_dim, stream ? static_cast<hipStream_t>(stream) : ctx->stream),
                    "prefill attention launch");
 }

@@ -22,7 +22,12 @@ struct PrefillAttnArgs {
   uint32_t* err;
   int nq, nkv, n, pos0;
   float scale;
+  float* part;        // scratch of part_bytes (16-byte aligned), or null
+  size_t part_bytes;
 };
+// Scratch with which few rows at a long context run on more CUs (0: they have
+// no such form); the results do not depend on it.
+size_t attn_prefill_scratch(int nq, int nkv, int head_dim, int n);
 // head_dim 64 or 128
 hipError_t launch_attn_prefill(const PrefillAttnArgs& a, int head_dim, hipStream_t st);
 
