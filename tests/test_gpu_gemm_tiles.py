@@ -22,11 +22,15 @@ def same_bits(a, b):
     return np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
-# narrow tiles: whole ones whose width is no multiple of 64, partial rows and
-# columns, one stage and a partial last stage; then the first width past them
+# few tiles: whole ones whose width is no multiple of 64, partial rows and
+# columns, one stage and a partial last stage, on the 32-row tile; then in_dims
+# from the narrow tile's 1024 (Q4_0) and 2048 (Q8_0) on, and the first below;
+# and the first width past the narrow tile
 @pytest.mark.parametrize("wt", [Q4_0, Q8_0])
 @pytest.mark.parametrize("il,m,n,k", [(4, 32, 96, 256), (1, 33, 100, 544), (4, 1, 4, 32), (1, 64, 1340, 512),
-                                      (4, 16, 8192, 256), (4, 16, 8256, 256)])
+                                      (4, 16, 8192, 256), (4, 16, 8256, 256), (4, 32, 96, 2048), (1, 33, 100, 2080),
+                                      (4, 1, 4, 2080), (1, 64, 1340, 2048), (4, 33, 100, 1024), (1, 17, 36, 1056),
+                                      (4, 33, 100, 992), (1, 17, 36, 2016), (4, 16, 8192, 2048), (4, 16, 8256, 2048)])
 def test_q8act_narrow_tiles(ctx, zo, wt, il, m, n, k):
     rng = np.random.default_rng(m + n + k + wt)
     w, x = synth.weight(rng, wt, n, k, il), synth.activations(rng, m * k).reshape(m, k)

@@ -761,10 +761,12 @@ zg_status zg::run_gemm(zg_ctx* ctx, const int8_t* qs, const uint16_t* xd, const 
   const size_t tiles32 = ((n + kBN - 1) / kBN) * ((m + 31) / 32);
   if (tiles64 >= (size_t)3 * gemm_cu_count()) {
     launch_gemm_il<64, ZG_GEMM_BK64, 256>(a, w_type, interleave, st);
-  } else if (tiles32 <= (size_t)gemm_cu_count() / 2) {
+  } else if (tiles32 <= (size_t)gemm_cu_count() / 2 && k >= (w_type == ZG_Q4_0 ? 1024u : 2048u)) {
     // half the CUs would be idle: 32 x 32 tiles, four waves (Q4_0X4 128 x 2048
-    // x 6144 20.7 -> 17.8 us, 64 x 4096 x 2048 8.2 -> 7.5 us; from one 32 x 64
-    // tile per CU on they lose, 128 x 4096 x 2048 8.5 against 9.1 us)
+    // x 6144 20.4 -> 17.7 us, 64 x 4096 x 2048 8.2 -> 7.5 us; from one 32 x 64
+    // tile per CU on they lose, 128 x 4096 x 2048 8.5 against 9.1 us, and so
+    // they do with few stages to gain on: Q8_0X4 300 x 256 x 512 4.1 against 4.8
+    // us, 16 x 4096 x 1056 6.2 against 7.2, Q4_0 32 x 6144 x 512 4.0 against 4.6)
     launch_gemm_il<32, 8, 256, 32>(a, w_type, interleave, st);
   } else {
     launch_gemm_il<32, 8, 512>(a, w_type, interleave, st);
